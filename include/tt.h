@@ -263,10 +263,12 @@ tt_status tt_scene_set_geometries(tt_scene *s, const tt_geometry *g, int32_t n);
  * FP64 total weight (sum of luminance * sin(theta) over texels). */
 tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double *total);
 
-/* Traversal launch tuning. variant: 0 = per-lane exact (single-lane order; hit ids
- * bit-identical to the host reference traversal), 1 = speculative while-while
- * (Aila-Laine postponed leaf + wave ballot). lds_stack: LDS stack entries per lane
- * (8, 16, 24 or 32); block: threads per block (64..256, multiple of 64).
+/* Traversal launch tuning. variant (scenes of short rays, which keep the two-child loop;
+ * elsewhere both give the same walk and records): 0 = per-lane exact (single-lane order;
+ * hit ids bit-identical to the host reference traversal), 1 = speculative while-while
+ * (Aila-Laine postponed leaf + wave ballot). lds_stack: LDS stack entries of 4 bytes per
+ * lane (8, 16, 24 or 32; a closest-hit entry of the four-child walk is 8 bytes, and 3/4 of
+ * the number of them are kept in LDS); block: threads per block (64..256, multiple of 64).
  * refill: 0 (default) = one wave per 64-ray group; 1..64 = persistent waves: the
  * launch holds as many waves as the GPU keeps resident, wave w of W traces the
  * 64-ray groups w, w + W, ..., and a lane whose ray is done takes the wave's next ray

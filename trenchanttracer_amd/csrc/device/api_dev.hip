@@ -97,6 +97,17 @@ static void scratch_setup(int device) {
     });
 }
 
+TraceArgs trace_args(const tt_scene *s) {
+    TraceArgs a{};
+    a.nodes = reinterpret_cast<const float4 *>(s->nodes);
+    a.tris = reinterpret_cast<const float4 *>(s->tris);
+    a.num_nodes = (int32_t)s->num_nodes;
+    a.wide = reinterpret_cast<const uint4 *>(s->wide);
+    a.wide_bound = s->wide_bound;
+    a.roots = s->roots;
+    return a;
+}
+
 }  // namespace tt
 
 extern "C" {
@@ -325,6 +336,14 @@ void tt_timer_destroy(tt_timer *t) {
 
 tt_status tt_scene_create(tt_ctx *ctx, const tt_mesh *mesh, const tt_bvh *bvh, const tt_material *mats, int32_t nmats,
                           const float *env_rgb, int32_t env_w, int32_t env_h, float env_scale, tt_scene **out) {
+    return create_scene(ctx, mesh, bvh, mats, nmats, env_rgb, env_w, env_h, env_scale, {}, out);
+}
+
+}  // extern "C"
+
+tt_status tt::create_scene(tt_ctx *ctx, const tt_mesh *mesh, const tt_bvh *bvh, const tt_material *mats, int32_t nmats,
+                           const float *env_rgb, int32_t env_w, int32_t env_h, float env_scale,
+                           const std::vector<int32_t> &roots, tt_scene **out) {
     if (!ctx || !bvh || !out) return fail(TT_ERR_INVALID, "tt_scene_create: null argument");
     if (nmats < 0 || (nmats > 0 && !mats)) return fail(TT_ERR_INVALID, "tt_scene_create: bad materials");
     if (env_rgb && (env_w <= 0 || env_h <= 0 || (int64_t)env_w * env_h > (1LL << 28)))
@@ -472,6 +491,8 @@ tt_status tt_scene_create(tt_ctx *ctx, const tt_mesh *mesh, const tt_bvh *bvh, c
     }
     if (nmats > 0) up((void **)&s->mats, mats, sizeof(tt_material) * (size_t)nmats, "scene materials");
     s->num_mats = nmats;
+    if (!roots.empty()) up((void **)&s->roots, roots.data(), roots.size() * 4, "scene roots");
+    if (st == TT_OK) st = build_wide(s, f.dev_nodes, roots.empty() ? std::vector<int32_t>{0} : roots);
     if (st == TT_OK && env_rgb) st = build_env(s, env_rgb, env_w, env_h, env_scale);
     if (st != TT_OK) {
         tt_scene_destroy(s);
@@ -481,6 +502,8 @@ tt_status tt_scene_create(tt_ctx *ctx, const tt_mesh *mesh, const tt_bvh *bvh, c
     return TT_OK;
 }
 
+extern "C" {
+
 void tt_scene_destroy(tt_scene *s) {
     if (!s) return;
     hipSetDevice(s->ctx->device);
@@ -488,7 +511,7 @@ void tt_scene_destroy(tt_scene *s) {
     free_render_state(s);
     void *ptrs[] = {s->nodes, s->tris, s->tri_normals, s->tri_mat, s->mats, s->tri_geo, s->shade_tri, s->emit_tri, s->emit_cdf,
                     s->emit_verts, s->env_rgb, s->env_marg_cdf, s->env_cond_cdf, s->env_pdf_scale, s->geoms,
-                    s->env_marg_cells, s->env_cells};
+                    s->env_marg_cells, s->env_cells, s->wide, s->roots};
     for (void *p : ptrs)
         if (p) hipFree(p);
     delete s;
@@ -534,14 +557,11 @@ static tt_status trace_impl(tt_scene *s, const tt_ray *rays, int64_t n, tt_hit *
     tt_status st = resolve_cfg(cfg, c);
     if (st != TT_OK) return st;
     if (n == 0) return TT_OK;
-    TraceArgs a{};
-    a.nodes = reinterpret_cast<const float4 *>(s->nodes);
-    a.tris = reinterpret_cast<const float4 *>(s->tris);
+    TraceArgs a = trace_args(s);
     a.rays = rays;
     a.hits = hits;
     a.flags = flags;
     a.n = n;
-    a.num_nodes = (int32_t)s->num_nodes;
     hipStream_t hs = stream ? (hipStream_t)stream : s->ctx->stream;
     TT_HIP(hipSetDevice(s->ctx->device), "hipSetDevice");
     if (c.reorder && noalloc) {
@@ -641,12 +661,9 @@ tt_status tt_bench_fetch_replay(tt_scene *s, const tt_ray *rays, int64_t n, cons
     tt_ctx *ctx = s->ctx;
     hipStream_t hs = ctx->stream;
     TT_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    TraceArgs a{};
-    a.nodes = reinterpret_cast<const float4 *>(s->nodes);
-    a.tris = reinterpret_cast<const float4 *>(s->tris);
+    TraceArgs a = trace_args(s);
     a.rays = rays;
     a.n = n;
-    a.num_nodes = (int32_t)s->num_nodes;
     if (c.reorder) {
         size_t need = 0, sort_bytes = 0;
         TT_HIP(reorder_workspace_bytes(n, &need, &sort_bytes), "fetch replay: reorder workspace size");

@@ -10,6 +10,7 @@ namespace tt {
 
 constexpr int kSentinel = 0x76543210;  // IntersectKernel.cuh:9
 constexpr int kStackCap = 72;          // >= 64 outstanding pushes (tree depth <= 64)
+constexpr int kWideCap = 48;           // entries of the wide walk's stack
 
 struct TraceArgs {
     const float4 *nodes;   // 4 float4 per node
@@ -19,7 +20,10 @@ struct TraceArgs {
     int32_t *flags;        // any-hit output (or nullptr)
     int64_t n;
     int32_t num_nodes;
-    const int32_t *ray_root;  // if set: root node of each ray (several scenes in one node array)
+    const uint4 *wide;        // four-child tree and its triangle records (nullptr: walk the two-child one)
+    float wide_bound;         // largest coordinate of a plane
+    const int32_t *ray_root;  // if set: scene of each ray (its root is that record of the wide tree)
+    const int32_t *roots;     // if set: the scenes' roots in the two-child tree
     const int32_t *n_dev;  // if set: ray count read on the device (capped at n)
     int32_t *reset0;       // if set: zeroed by the first lane of block 0
     int32_t *reset1;

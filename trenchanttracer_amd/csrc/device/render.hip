@@ -35,7 +35,7 @@ struct RenderState {
     int32_t cap = 0;
     tt_ray *rays[2] = {nullptr, nullptr};
     int32_t *path[2] = {nullptr, nullptr};
-    int32_t *root[2] = {nullptr, nullptr};   // root node of each queued ray's scene
+    int32_t *root[2] = {nullptr, nullptr};   // scene of each queued ray
     // next-event queues of even and odd bounces (a bounce's shadow work may still run
     // while the next bounce fills the other set)
     int32_t *sroot[2] = {nullptr, nullptr};
@@ -144,7 +144,7 @@ struct CamArgs {
 };
 
 // Up to kMaxScenes scenes rendered in one wavefront: per scene its pixel range
-// in the concatenated image, resolution, root node and camera.
+// in the concatenated image, resolution and camera.
 constexpr int kMaxScenes = 64;
 // Path slots walk 8x8 pixel tiles: on the 1080p path-trace case (64 spp, depth 16,
 // sample-major path ids) the render took 0.1605 s against 0.1650 s in pixel-row
@@ -154,7 +154,7 @@ struct SceneTable {
     int32_t n;
     int32_t tile;   // slot order inside a scene: 0 = pixel rows, T > 1 = T x T tiles
     int32_t pix_off[kMaxScenes + 1];
-    int32_t w[kMaxScenes], h[kMaxScenes], root[kMaxScenes];
+    int32_t w[kMaxScenes], h[kMaxScenes];
     CamArgs cam[kMaxScenes];
 };
 
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a) {
     f3 d = vnorm(vnorm(on_image - ap));
     a.rays[p] = {ap.x, ap.y, ap.z, a.tmin, d.x, d.y, d.z, 1e20f};
     a.path[p] = p;
-    a.root[p] = a.tab->root[sid];
+    a.root[p] = sid;
     // reference mode: mask and path radiance. Path mode starts every path from
     // throughput 1 and roulette weight 1, which its camera-bounce shading takes as
     // constants (every generated path is in that bounce's queue), so nothing is
@@ -1809,13 +1809,10 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     const unsigned gblocks =
         (unsigned)std::min<int64_t>(((int64_t)cap + 255) / 256, 16LL * std::max(1, s->ctx->num_cus));
     const unsigned sblocks = (unsigned)(((int64_t)cap + kAppendBlock - 1) / kAppendBlock);
-    TraceArgs ta{};
-    ta.nodes = (const float4 *)s->nodes;
-    ta.tris = (const float4 *)s->tris;
+    TraceArgs ta = trace_args(s);
     ta.rays = rs->rays[cur];
     ta.hits = rs->hits;
     ta.n = cap;
-    ta.num_nodes = (int32_t)s->num_nodes;
     ta.n_dev = rs->counts + cur;
     ta.reset0 = rs->counts + nxt;
     ta.reset1 = rs->counts + sc;
@@ -1904,13 +1901,10 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     if (e == hipSuccess && as) e = hipStreamWaitEvent(as, s->ctx->shade_done, 0);
     if (e != hipSuccess) return e;
     const hipStream_t ss = as ? as : hs;
-    TraceArgs sh{};
-    sh.nodes = (const float4 *)s->nodes;
-    sh.tris = (const float4 *)s->tris;
+    TraceArgs sh = trace_args(s);
     sh.rays = rs->srays[set];
     sh.flags = rs->socc[set];
     sh.n = cap;
-    sh.num_nodes = (int32_t)s->num_nodes;
     sh.n_dev = rs->counts + sc;
     sh.ray_root = rs->sroot[set];
     e = launch_trace(sh, variant, true, lds, block, 0, refill_later, s->ctx->num_cus, ss, kTriTwoSided);
@@ -2088,8 +2082,8 @@ hipError_t guide_train_pass(GuideRun *gr, int32_t max_depth, hipStream_t hs) {
     return e;
 }
 
-// Renders nsc scenes sharing one node / triangle array (roots[k] = root node of
-// scene k) in one wavefront. out: host, concatenated images in scene order.
+// Renders nsc scenes sharing one node / triangle array in one wavefront. out: host,
+// concatenated images in scene order.
 // Where a render's image goes: `count` floats (and FP64 values, if rgb64 is set) of
 // the concatenated image starting at `offset`.
 struct OutSeg {
@@ -2098,9 +2092,8 @@ struct OutSeg {
     int64_t offset, count;
 };
 
-tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const int32_t *roots,
-                      const tt_render_params *p, const OutSeg *segs, int32_t nseg, tt_render_stats *stats,
-                      GuideRun *gr = nullptr) {
+tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const tt_render_params *p, const OutSeg *segs,
+                      int32_t nseg, tt_render_stats *stats, GuideRun *gr = nullptr) {
     tt_status st = validate_params(p);
     if (st != TT_OK) return st;
     if (gr && p->mode != TT_RENDER_PATH) return fail(TT_ERR_INVALID, "render: guiding needs path mode");
@@ -2119,7 +2112,6 @@ tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const int
         tab.pix_off[k] = (int32_t)npix64;
         tab.w[k] = c.width;
         tab.h[k] = c.height;
-        tab.root[k] = roots[k];
         tab.cam[k] = camera_args(c, p->pi, p->two_pi);
         npix64 += (int64_t)c.width * c.height;
     }
@@ -2342,10 +2334,9 @@ tt_status tt_camera_from_orbit(const float center[3], float yaw, float pitch, fl
 tt_status tt_render(tt_scene *s, const tt_camera *cam, const tt_render_params *p, float *rgb_out, double *rgb64_out,
                     tt_render_stats *stats) {
     if (!s || !cam || !p || !rgb_out) return fail(TT_ERR_INVALID, "tt_render: null argument");
-    const int32_t root = 0;
     const int64_t n3 = (int64_t)std::max(0, cam->width) * std::max(0, cam->height) * 3;
     const OutSeg seg{rgb_out, rgb64_out, 0, n3};
-    return render_impl(s, 1, cam, &root, p, &seg, 1, stats);
+    return render_impl(s, 1, cam, p, &seg, 1, stats);
 }
 
 tt_status tt_guide_render(tt_scene *s, tt_guide *g, const tt_camera *cam, const tt_render_params *p,
@@ -2370,10 +2361,9 @@ tt_status tt_guide_render(tt_scene *s, tt_guide *g, const tt_camera *cam, const 
     gr.max_bounce = gp->max_bounce;
     gr.growth = std::max(1, gp->pass_growth);
     gr.gd.learn_alpha = gp->learn_alpha ? 1 : 0;
-    const int32_t root = 0;
     const int64_t n3 = (int64_t)std::max(0, cam->width) * std::max(0, cam->height) * 3;
     const OutSeg seg{rgb_out, rgb64_out, 0, n3};
-    tt_status st = render_impl(s, 1, cam, &root, &q, &seg, 1, stats, &gr);
+    tt_status st = render_impl(s, 1, cam, &q, &seg, 1, stats, &gr);
     if (st == TT_OK && gstats) {
         gstats->train_steps = gr.steps;
         gstats->train_rows = gr.rows;
@@ -2438,8 +2428,8 @@ tt_status tt_batch_create(tt_ctx *ctx, int32_t n, const tt_mesh *const *meshes, 
                 F.dev_tris.insert(F.dev_tris.end(), r, r + 12);
             }
         }
-        tt_status st = tt_scene_create(ctx, b->mesh, b->bvh, allm.data(), (int32_t)allm.size(), env_rgb, env_w, env_h,
-                                       env_scale, &b->scene);
+        tt_status st = create_scene(ctx, b->mesh, b->bvh, allm.data(), (int32_t)allm.size(), env_rgb, env_w, env_h,
+                                    env_scale, b->roots, &b->scene);
         if (st != TT_OK) {
             tt_batch_destroy(b.release());
             return st;
@@ -2472,7 +2462,7 @@ tt_status tt_batch_render(tt_batch *b, const tt_camera *cams, const tt_render_pa
         segs[(size_t)k] = OutSeg{rgb_out[k], nullptr, off, cnt};
         off += cnt;
     }
-    return render_impl(b->scene, n, cams, b->roots.data(), p, segs.data(), n, stats);
+    return render_impl(b->scene, n, cams, p, segs.data(), n, stats);
 }
 
 tt_status tt_debug_bsdf_sample(tt_ctx *ctx, const tt_material *m, const float wo[3], int32_t front, int64_t n,

@@ -39,6 +39,9 @@ struct tt_scene {
     void *tris = nullptr;        // float4 x 3 per triangle record
     int64_t num_nodes = 0;
     int64_t num_tris = 0;
+    void *wide = nullptr;        // the four-child tree the traversal walks, with its triangle records (wide.hip)
+    float wide_bound = 0.0f;
+    int32_t *roots = nullptr;    // several scenes in one tree: their two-child roots
     // shading data by original triangle id
     void *tri_normals = nullptr;  // float4 x 3 per triangle
     int32_t *tri_mat = nullptr;
@@ -78,6 +81,13 @@ struct tt_timer {
 
 namespace tt {
 tt_status dev_alloc(tt_ctx *ctx, void **p, size_t bytes, const char *what);
+tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const std::vector<int32_t> &roots);
+// tt_scene_create for several trees in one node array (roots: their root nodes)
+tt_status create_scene(tt_ctx *ctx, const tt_mesh *mesh, const tt_bvh *bvh, const tt_material *mats, int32_t nmats,
+                       const float *env_rgb, int32_t env_w, int32_t env_h, float env_scale,
+                       const std::vector<int32_t> &roots, tt_scene **out);
+struct TraceArgs;
+TraceArgs trace_args(const tt_scene *s);   // the scene's trees
 tt_status build_env(tt_scene *s, const float *rgb, int32_t w, int32_t h, float scale);
 void free_render_state(tt_scene *s);
 }  // namespace tt

@@ -1,31 +1,43 @@
 // Closest-hit / any-hit traversal of the SBVH on gfx950 (wave64).
 //
-// Per lane: one ray at a time (a lane whose ray is done takes the next one of its
-// wave's sequence), the while-while loop of Aila & Laine ("Understanding the
-// Efficiency of Ray Traversal on GPUs", HPG 2009) in the form of the reference
-// intersect() (include/geometry/IntersectKernel.cuh:78-296):
+// k_trace_wide walks the four-child tree of wide.hip (48-byte nodes, planes quantised to
+// 8 bits, always outwards) and tests every triangle with the reference's arithmetic. Its
+// results are those of the reference intersect() (include/geometry/IntersectKernel.cuh:
+// 78-296) on the two-child tree, which walk_exact and k_trace restate:
 //   - ray precompute idir / ood with the 2^-80 clamp                (:92-101)
 //   - two child boxes per 64-byte node, slab entry/exit as 3-operand integer
 //     min/max of the float bit patterns (v_min3_i32 / v_max3_i32 restate the
 //     PTX vmin/vmax.s32 forms), traverse iff entry <= exit, entry >= tmin,
 //     entry <= 1e20                                                  (:126-147)
 //   - near child first, far child pushed                             (:149-167)
-//   - first leaf postponed                                           (:172-178)
-//   - Möller–Trumbore on v0 and the two edges, front faces only with
+//   - Moeller-Trumbore on v0 and the two edges, front faces only with
 //     |det| > 1e-5, tmin < t < best                                  (:230-257)
-// Arithmetic is unfused (fp contract off) and division IEEE, so for a given
+// Arithmetic of these is unfused (fp contract off) and division IEEE, so for a given
 // visiting order every decision is bit-identical to the host restatement.
 //
-// Two loop variants:
-//   VARIANT 0 (exact): a lane leaves the node loop as soon as it holds a leaf,
-//     i.e. the single-lane order. Hit ids, t, u, v are bit-identical to the
-//     host traversal of the same tree.
-//   VARIANT 1 (speculative): lanes keep descending until no lane of the wave is
-//     still searching for its first leaf (__any ballot, :192-203). Results differ
-//     from the single-lane order only where a triangle lies on a box boundary
-//     within rounding of the current hit distance.
-// Stack: the top kLds entries of each lane live in LDS ([entry][lane] so the
-// lanes of a wave hit distinct banks), deeper entries in per-lane scratch.
+// Why the wide walk gives the same hits. The two-child walk tests the triangles of the
+// leaves whose boxes the ray enters (a leaf's box lies inside every ancestor's, checked
+// when the wide tree is built, and rounding is monotone, so passing the leaf's slab test
+// implies passing its ancestors'). The wide boxes contain the two-child ones by more
+// than the rounding of both slab tests, so the wide walk tests at least those triangles.
+// When a ray is done its winner's leaf box is put through the two-child slab test at the
+// distance of the nearest other triangle (next_t): if it passes, the two-child walk enters
+// that leaf whatever its best distance was by then, and no tested triangle is nearer. If it
+// does not pass (a hit within rounding of its box's edge), or two triangles tie exactly
+// (the first one visited wins there), or the ray is one the quantised arithmetic does not
+// cover (non-finite or overflowing terms, negative tmin, a full stack), the lane walks the
+// two-child tree. An any-hit ray applies the leaf test to every triangle it would accept.
+// (Boxes are culled against the best distance with 2^-10 to spare: a triangle whose
+// computed t lies further than that below its own box could still be skipped.)
+//
+// Stack: the lowest S entries of each lane live in LDS ([entry][lane] so the lanes of a
+// wave hit distinct banks), deeper entries in per-lane scratch.
+//
+// k_trace is the two-child while-while loop of Aila & Laine ("Understanding the Efficiency
+// of Ray Traversal on GPUs", HPG 2009): for scenes without a four-child tree, and, with
+// recording, for the node-fetch probe.
+#include <type_traits>
+
 #include "dev_common.h"
 
 #pragma clang fp contract(off)
@@ -80,12 +92,474 @@ struct Stack {
     }
 };
 
-// REC (closest hit only; the node-fetch probe): 1 counts each ray's node visits,
-// triangle tests and leaf visits; 2 records at every node visit the slab test's
-// outcome as a 4-bit code (bit 0: child 0 entered, bit 1: child 1 entered, bit 2:
-// both, child 1 first); 3 replays: the same loop, stack, leaf postponement, ballots
-// and refills, every node and triangle record fetched, but each node's outcome read
-// from the record instead of computed and no triangle arithmetic.
+// One child box of a two-child node against a ray (IntersectKernel.cuh:126-147).
+struct RayTerms {
+    float idirx, idiry, idirz, oodx, oody, oodz, tmin;
+};
+__device__ __forceinline__ bool slab(float4 xy, float zlo, float zhi, const RayTerms &r, float hit_t, float *entry) {
+    const float lox = xy.x * r.idirx - r.oodx, hix = xy.y * r.idirx - r.oodx;
+    const float loy = xy.z * r.idiry - r.oody, hiy = xy.w * r.idiry - r.oody;
+    const float loz = zlo * r.idirz - r.oodz, hiz = zhi * r.idirz - r.oodz;
+    const float cmin = span_begin(lox, hix, loy, hiy, loz, hiz, r.tmin);
+    const float cmax = span_end(lox, hix, loy, hiy, loz, hiz, hit_t);
+    const float ray_tmax = 1e20f;
+    *entry = cmin;
+    return (cmin <= cmax) && (cmin >= r.tmin) && (cmin <= ray_tmax);
+}
+
+// Moeller-Trumbore, IntersectKernel.cuh:230-254 (edges precomputed: same bits): whether
+// the triangle is crossed at a t in (tmin, tbest], with that t and the barycentrics.
+template <int TRI>
+__device__ __forceinline__ bool tri_test(float4 A, float4 B, float4 C, float ox, float oy, float oz, float dx, float dy,
+                                         float dz, float tmin, float tbest, float *t_out, float *u_out, float *v_out) {
+    const float tvx = ox - A.x, tvy = oy - A.y, tvz = oz - A.z;
+    const float pvx = dy * C.z - dz * C.y;
+    const float pvy = dz * C.x - dx * C.z;
+    const float pvz = dx * C.y - dy * C.x;
+    const float det = B.x * pvx + B.y * pvy + B.z * pvz;
+    const float inv = 1.0f / det;
+    const float u = (tvx * pvx + tvy * pvy + tvz * pvz) * inv;
+    const float qvx = tvy * B.z - tvz * B.y;
+    const float qvy = tvz * B.x - tvx * B.z;
+    const float qvz = tvx * B.y - tvy * B.x;
+    const float v = (dx * qvx + dy * qvy + dz * qvz) * inv;
+    const float t = (C.x * qvx + C.y * qvy + C.z * qvz) * inv;
+    // bitwise: every lane takes the same instructions (short-circuit branches cost more
+    // than the comparisons they skip)
+    bool ok;
+    if (TRI == kTriReference) {
+        const float EPS = 0.00001f;
+        // the reference's back-face bounds (IntersectKernel.cuh:248-250) have their
+        // comparisons reversed, !(u > 0 || u < 1) && !(v > 0 || u + v < 1): they hold for
+        // a NaN u alone
+        ok = (bool)(((int)(det > EPS) & (int)!(u < 0.0f) & (int)!(u > 1.0f) & (int)!(v < 0.0f) & (int)!((u + v) > 1.0f)) |
+                    ((int)(det < -EPS) & (int)(u != u) & (int)!(v > 0.0f)));
+    } else {
+        ok = (bool)((int)(det != 0.0f) & (int)(u >= 0.0f) & (int)(u <= 1.0f) & (int)(v >= 0.0f) & (int)((u + v) <= 1.0f));
+    }
+    *t_out = t;
+    *u_out = u;
+    *v_out = v;
+    return (bool)((int)ok & (int)(tmin < t) & (int)(t <= tbest));
+}
+
+// ------------------------------------------------------------------ the traversal
+// Stack of a lane: entries of E (closest hit: entry distance and child, so that a popped
+// subtree past the best hit is dropped unread; any hit: the child alone), the lowest S in
+// LDS ([entry][lane]: the lanes of a wave hit distinct banks), deeper ones in per-lane
+// scratch. Entries past kWideCap are not kept: push tells, and the lane walks the two-child
+// tree instead. The LDS pointers keep their address space: through a generic one the
+// compiler merges the two reads of pop into one flat load of a selected address.
+#define TT_LDS __attribute__((address_space(3)))
+template <class E, int S>
+struct WideStack {
+    TT_LDS E *bottom, *top;   // the lane's column; the first free LDS entry
+    int stride;
+    int over;                 // entries in scratch
+    E *spill;
+    __device__ __forceinline__ bool empty() const { return top == bottom; }
+    __device__ __forceinline__ void clear() {
+        top = bottom;
+        over = 0;
+    }
+    // up to three entries, the last valid one on top: written unconditionally, each over
+    // the one before where that was not valid (some lane of a wave nearly always pushes,
+    // so branches around the writes save nothing). False: one was not kept.
+    __device__ __forceinline__ bool push3(E a, bool va, E b, bool vb, E c, bool vc) {
+        if (top <= bottom + (S - 3) * stride) {
+            top[0] = a;
+            top += va ? stride : 0;
+            top[0] = b;
+            top += vb ? stride : 0;
+            top[0] = c;
+            top += vc ? stride : 0;
+            return true;
+        }
+        bool kept = true;
+        if (va) kept = push(a);
+        if (vb) kept = push(b) && kept;
+        if (vc) kept = push(c) && kept;
+        return kept;
+    }
+    __device__ __forceinline__ bool push(E v) {
+        if (top < bottom + S * stride) {
+            top[0] = v;
+            top += stride;
+        } else if (over < kWideCap - S) {
+            spill[over++] = v;
+        } else {
+            return false;
+        }
+        return true;
+    }
+    __device__ __forceinline__ E pop() {   // not empty
+        E e = top[-stride];
+        if (over == 0) top -= stride;
+        else e = spill[--over];
+        return e;
+    }
+};
+
+struct HitState {
+    float t, u, v;
+    int id;
+};
+
+// The two-child walk of one ray in the single-lane order, on the lane's own stack memory.
+template <bool ANY, int S, int TRI>
+__device__ __forceinline__ void walk_exact(const TraceArgs &a, int root, float ox, float oy, float oz, float dx, float dy,
+                                           float dz, const RayTerms &r, float tmax, int *lds, int stride, int *spill,
+                                           HitState &h) {
+    Stack<S> st{lds, stride, 0, 0, spill};
+    h = HitState{tmax, 0.0f, 0.0f, -1};
+    int node = root, leaf = 0;
+    while (node != kSentinel) {
+        while (node >= 0 && node != kSentinel) {
+            const float4 *np = a.nodes + (int64_t)node * 4;
+            const float4 n0 = np[0], n1 = np[1], nz = np[2];
+            const int2 ch = reinterpret_cast<const int2 *>(np + 3)[0];
+            float e0, e1;
+            const bool t0 = slab(n0, nz.x, nz.y, r, h.t, &e0);
+            const bool t1 = slab(n1, nz.z, nz.w, r, h.t, &e1);
+            if (!t0 && !t1) {
+                node = st.pop();
+            } else {
+                int far = ch.y;
+                node = t0 ? ch.x : ch.y;
+                if (t0 && t1) {
+                    if (e1 < e0) {
+                        far = node;
+                        node = ch.y;
+                    }
+                    st.push(far);
+                }
+            }
+            if (node < 0) {
+                leaf = node;
+                node = st.pop();
+                break;
+            }
+        }
+        while (leaf < 0) {
+            for (int tri = ~leaf;; ++tri) {
+                const float4 *tp = a.tris + (int64_t)tri * 3;
+                const float4 A = tp[0], B = tp[1], C = tp[2];
+                float t, u, v;
+                if (tri_test<TRI>(A, B, C, ox, oy, oz, dx, dy, dz, r.tmin, h.t, &t, &u, &v) && t < h.t) {
+                    h = HitState{t, u, v, fb(A.w)};
+                    if (ANY) return;
+                }
+                if (fb(C.w) != 0) break;
+            }
+            leaf = node;
+            if (node < 0) node = st.pop();
+        }
+    }
+}
+
+// Whether the two-child walk enters a leaf (its place: node * 2 + child) at best distance
+// hit_t.
+__device__ __forceinline__ bool in_leaf(const TraceArgs &a, int place, const RayTerms &r, float hit_t) {
+    const float4 *np = a.nodes + (int64_t)(place >> 1) * 4;
+    const float4 xy = np[place & 1];
+    const float2 z = reinterpret_cast<const float2 *>(np + 2)[place & 1];
+    float e;
+    return slab(xy, z.x, z.y, r, hit_t, &e);
+}
+
+// Whether the two-child walk reaches the triangle of a record, found in the leaf at
+// `place`, while its best distance is t or more, through any of its leaves: the records of
+// one triangle form a ring (a spatial split puts a triangle in several leaves, and the one
+// it was found in here may be one whose own box the ray misses: 1-3% of the soup's rays).
+// Longer rings than the limit go to the full walk.
+__device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, const RayTerms &r, float t) {
+    if (in_leaf(a, place, r, t)) return true;
+    int at = rec;
+    for (int i = 0; i < 16; ++i) {
+        at = fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[2].w) & 0x7FFFFFFF;
+        if (at == rec) return false;
+        if (in_leaf(a, fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[1].w), r, t)) return true;
+    }
+    return false;
+}
+
+// Four-child walk. What bounds it: VALU issue first, vector memory lane loads second. On
+// the 1M-triangle soup (8.3M rays in Morton order) the two-child while-while loop kept VALU
+// issue 90% and the address path 82% busy, with 32% of the lanes active: 1.85e9 VALU
+// instructions, 1.53e9 cache accesses and 4.0 ms a launch. Visiting four boxes with 3 loads
+// instead of 8, and taking node visits and triangle tests by the vote below (59% of the
+// lanes active), takes 1.45e9, 1.04e9 and 3.0 ms; each alone gains little, as the other
+// limit holds (four children in the while-while loop: 6.6 ms, slower).
+template <bool ANY, int S, int TRI>
+__global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
+    using E = typename std::conditional<ANY, int, uint64_t>::type;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    // XCD-contiguous order: the hardware hands blocks to the 8 XCDs round-robin, so
+    // block b runs on XCD b % 8; renumbering b -> (b % 8) * q + b / 8 (for the first
+    // 8q blocks, q = blocks / 8; the tail keeps its number) is a bijection that gives
+    // each XCD's L2 one contiguous range of waves
+    unsigned vb = blockIdx.x;
+    if (a.xcd_order) {
+        const unsigned q = gridDim.x >> 3;
+        if (vb < (q << 3)) vb = (vb & 7u) * q + (vb >> 3);
+    }
+    uint32_t n = (uint32_t)a.n;   // below 2^31 (launch_trace)
+    if (a.n_dev) n = min((uint32_t)max(0, *a.n_dev), n);
+    if (blockIdx.x == 0 && tid == 0) {
+        if (a.reset0) *a.reset0 = 0;
+        if (a.reset1) *a.reset1 = 0;
+    }
+    // Persistent waves (Aila & Laine's persistent threads with ray replacement):
+    // the grid holds about as many waves as the chip keeps resident, and wave w of W
+    // owns the 64-ray groups w, w + W, w + 2W, ... in that order, so that all waves
+    // sweep the ray range together (the rays in flight at any moment lie in a window
+    // of about 2W groups, as with one block per group, which keeps coherent rays'
+    // nodes in cache). A lane whose ray is done writes its result and takes the next
+    // ray of its wave's sequence (ballot and prefix count, no atomics): the lanes
+    // stay busy until the sequence runs out, instead of idling behind the wave's
+    // longest ray. Each ray's traversal is the same as with one ray per lane. The wave's
+    // number is read from its first lane, so that everything uniform stays in scalar
+    // registers and the loops below branch on scalars.
+    const uint32_t groups = (n + 63u) >> 6;
+    const uint32_t waves = max(1u, min(gridDim.x * (blockDim.x >> 6), groups));
+    const uint32_t w = vb * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
+    if (w >= waves) return;   // whole waves only: nothing below synchronises the block
+    const uint32_t total = ((groups - w + waves - 1u) / waves) * 64u;   // the wave's sequence positions
+    const unsigned long long below = (1ull << lane) - 1ull;
+
+    // one private array serves both walks
+    constexpr int kWideWords = (kWideCap - S) * (int)(sizeof(E) / 4);
+    constexpr int kSpillWords = kWideWords > kStackCap - S ? kWideWords : kStackCap - S;
+    __align__(8) int spill[kSpillWords];
+    WideStack<E, S> st;
+    st.bottom = (TT_LDS E *)lds_raw + tid;
+    st.stride = blockDim.x;
+    st.clear();
+    st.spill = reinterpret_cast<E *>(spill);
+
+    int rid = -1;              // the lane's ray (-1: none)
+    uint32_t cursor = 0;       // next sequence position (uniform)
+    float ox = 0.0f, oy = 0.0f, oz = 0.0f, tmin = 0.0f, dx = 0.0f, dy = 0.0f, dz = 1.0f;
+    float idirx = 0.0f, idiry = 0.0f, idirz = 0.0f;
+    float nearx = 0.0f, neary = 0.0f, nearz = 0.0f;   // -(o idir) less the rounding allowance
+    float farx = 0.0f, fary = 0.0f, farz = 0.0f;      // -(o idir) plus it
+    int node = kSentinel;      // inner node to visit; sign set: a leaf waiting for room; kSentinel: none
+    int leaf = 0, leaf2 = 0;   // sign set: next record of the leaf being tested, first of the one after it
+    float hit_t = 0.0f;
+    int cull = 0;              // bits of the distance boxes are culled against (hit_t and 2^-10 to spare)
+    // the winner's record (-1: none; any hit: 0 once occluded). Its id and barycentrics go
+    // straight to the ray's hit record when it is accepted, which frees their registers.
+    int hit_rec = -1, hit_place = 0;   // (and the place of its leaf)
+    float next_t = 0.0f;       // no other accepted triangle lies below this (at most where boxes are culled)
+    bool redo = false;         // not for the wide walk
+
+    for (;;) {
+        const bool done = node == kSentinel && st.empty() && leaf >= 0;
+        if (done && rid >= 0) {
+            const RayTerms r{idirx, idiry, idirz, ox * idirx, oy * idiry, oz * idirz, tmin};
+            bool walk = redo;
+            if (!ANY && !walk && hit_rec >= 0)
+                walk = !(hit_t < next_t) || !reached(a, hit_rec, hit_place, r, fminf(next_t, bf(cull)));
+            if (walk) {
+                HitState h;
+                walk_exact<ANY, S, TRI>(a, a.roots ? a.roots[a.ray_root ? a.ray_root[rid] : 0] : 0, ox, oy, oz, dx, dy, dz,
+                                        r, a.rays[rid].tmax, reinterpret_cast<int *>(lds_raw) + tid * (int)(sizeof(E) / 4),
+                                        st.stride * (int)(sizeof(E) / 4), spill, h);
+                if (ANY) hit_rec = h.id == -1 ? -1 : 0;
+                else *reinterpret_cast<float4 *>(a.hits + rid) = make_float4(bf(h.id), h.t, h.u, h.v);
+            }
+            if (ANY) a.flags[rid] = hit_rec >= 0 ? 1 : 0;
+            else if (!walk && hit_rec < 0)
+                *reinterpret_cast<float4 *>(a.hits + rid) = make_float4(bf(-1), hit_t, 0.0f, 0.0f);
+            rid = -1;
+        }
+        const unsigned long long m = __ballot(done);
+        // new rays once enough lanes are idle (all idle always qualifies, so the
+        // wave cannot wait on itself)
+        const bool take = (int32_t)__popcll(m) >= a.refill;
+        if (take && done) {
+            const uint32_t q = cursor + (uint32_t)__popcll(m & below);
+            if (q < total) {
+                const uint32_t r = ((q >> 6) * waves + w) * 64u + (q & 63u);
+                if (r < n) rid = (int)(a.order ? a.order[r] : r);
+            }
+            if (rid >= 0) {
+                const float4 *rp = reinterpret_cast<const float4 *>(a.rays + rid);
+                const float4 r0 = rp[0], r1 = rp[1];
+                ox = r0.x;
+                oy = r0.y;
+                oz = r0.z;
+                tmin = r0.w;
+                dx = r1.x;
+                dy = r1.y;
+                dz = r1.z;
+                const float tmax = r1.w;
+                const float ooeps = 0x1p-80f;
+                idirx = 1.0f / (fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
+                idiry = 1.0f / (fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
+                idirz = 1.0f / (fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
+                // allowance for the rounding of both slab tests (wide.hip's planes are exact
+                // to 2^-53): the two-child test's terms are off by at most
+                // 2.01 (B + |o|) |idir| 2^-24 and this one's by 4.1 of the same, B the largest
+                // coordinate of a plane; 8 covers the two
+                const float sx = (fabsf(ox) + a.wide_bound) * fabsf(idirx) * 0x1p-21f;
+                const float sy = (fabsf(oy) + a.wide_bound) * fabsf(idiry) * 0x1p-21f;
+                const float sz = (fabsf(oz) + a.wide_bound) * fabsf(idirz) * 0x1p-21f;
+                nearx = -(ox * idirx) - sx;
+                neary = -(oy * idiry) - sy;
+                nearz = -(oz * idirz) - sz;
+                farx = sx - ox * idirx;
+                fary = sy - oy * idiry;
+                farz = sz - oz * idirz;
+                // rays the wide walk covers: all terms finite (NaN compares false), the
+                // allowance positive, distances that compare as integers
+                const bool fits = sx > 0.0f && sy > 0.0f && sz > 0.0f && sx < 1e30f && sy < 1e30f &&
+                                  sz < 1e30f && fb(tmin) >= 0 && tmin < 1e30f && fb(tmax) >= 0 && tmax <= INFINITY;
+                st.clear();
+                redo = !fits;
+                leaf = leaf2 = 0;
+                node = fits ? 3 * (a.ray_root ? a.ray_root[rid] : 0) : kSentinel;
+                hit_t = next_t = tmax;
+                hit_rec = -1;
+                cull = fb(tmax * 1.0009765625f);
+            }
+        }
+        if (take) cursor += (uint32_t)__popcll(m);
+        // ends once the sequence is used up and no lane holds a ray (only the last
+        // group of the range can be partial)
+        if (cursor >= total && __ballot(rid >= 0) == 0) break;
+        const int quit = cursor < total ? a.refill : 64;   // idle lanes at which the wave retires rays
+
+        // Each round the wave visits a node or tests a triangle, whichever more of its lanes
+        // are ready for (a node visit takes about twice a test's instructions, so it needs
+        // 1.4 times the lanes). Lanes hold up to two leaves, so most are ready for either.
+        // Simulated wave utilisation on Morton-sorted incoherent rays of 1M-triangle soup:
+        // 0.69 / 0.49 (node / triangle rounds) against 0.42 / 0.33 for the while-while loop,
+        // which runs each phase until its slowest lane is through.
+        for (;;) {
+            if (node == kSentinel && !st.empty()) {
+                const E e = st.pop();
+                if constexpr (ANY) node = e;
+                else node = (int)(e >> 32) <= cull ? (int)(uint32_t)e : kSentinel;
+            }
+            {
+                // a waiting leaf moves up where there is room
+                const bool move = (int)(node < 0) & (int)(leaf2 >= 0), first = leaf >= 0;
+                const int moved = node;
+                node = move ? kSentinel : node;
+                leaf2 = move ? (first ? 0 : moved) : leaf2;
+                leaf = (int)move & (int)first ? moved : leaf;
+            }
+            // records are 16-byte units below 2^30: an inner node compares below, kSentinel
+            // and leaves (sign set) above
+            const bool at_node = (uint32_t)node < (1u << 30), at_leaf = leaf < 0;
+            const unsigned long long mn = __ballot(at_node), mt = __ballot(at_leaf);
+            // (a lane that popped a stale entry counts as idle for this round)
+            if (64 - (int)__popcll(mn | mt) >= quit) break;
+            if ((int)__popcll(mn) * 5 >= (int)__popcll(mt) * 7) {
+                if (at_node) {
+                    const uint4 *np = a.wide + (uint32_t)node;
+                    const uint4 q0 = np[0], q1 = np[1], q2 = np[2];
+                    // plane scales 2^code, codes signed bytes
+                    const float kx = ldexpf(idirx, __builtin_amdgcn_sbfe((int)q1.y, 0, 8));
+                    const float ky = ldexpf(idiry, __builtin_amdgcn_sbfe((int)q1.y, 8, 8));
+                    const float kz = ldexpf(idirz, __builtin_amdgcn_sbfe((int)q1.y, 16, 8));
+                    const float bx = bf((int)q0.x), by = bf((int)q0.y), bz = bf((int)q0.z);
+                    const float nx = __builtin_fmaf(bx, idirx, nearx), fx = __builtin_fmaf(bx, idirx, farx);
+                    const float ny = __builtin_fmaf(by, idiry, neary), fy = __builtin_fmaf(by, idiry, fary);
+                    const float nz = __builtin_fmaf(bz, idirz, nearz), fz = __builtin_fmaf(bz, idirz, farz);
+                    const bool px = idirx >= 0.0f, py = idiry >= 0.0f, pz = idirz >= 0.0f;
+                    const uint32_t nwx = px ? q1.z : q1.w, fwx = px ? q1.w : q1.z;
+                    const uint32_t nwy = py ? q2.x : q2.y, fwy = py ? q2.y : q2.x;
+                    const uint32_t nwz = pz ? q2.z : q2.w, fwz = pz ? q2.w : q2.z;
+                    // per slot: entry distance with 8 times the slot in its low five bits (all
+                    // ones: not entered)
+                    uint32_t key[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float tnx = __builtin_fmaf((float)((nwx >> (8 * k)) & 255u), kx, nx);
+                        const float tny = __builtin_fmaf((float)((nwy >> (8 * k)) & 255u), ky, ny);
+                        const float tnz = __builtin_fmaf((float)((nwz >> (8 * k)) & 255u), kz, nz);
+                        const float tfx = __builtin_fmaf((float)((fwx >> (8 * k)) & 255u), kx, fx);
+                        const float tfy = __builtin_fmaf((float)((fwy >> (8 * k)) & 255u), ky, fy);
+                        const float tfz = __builtin_fmaf((float)((fwz >> (8 * k)) & 255u), kz, fz);
+                        // bits compare as the floats do: the entry is at least tmin >= +0, and a
+                        // negative exit stays negative
+                        const int en = max(max(fb(tnx), fb(tny)), max(fb(tnz), fb(tmin)));
+                        const int ex = min(min(fb(tfx), fb(tfy)), min(fb(tfz), cull));
+                        key[k] = en <= ex ? ((uint32_t)en & ~31u) | (uint32_t)(8 * k) : 0xFFFFFFFFu;
+                    }
+                    // nearest first
+                    const auto order2 = [&](int i, int j) {
+                        const uint32_t lo = min(key[i], key[j]), hi = max(key[i], key[j]);
+                        key[i] = lo;
+                        key[j] = hi;
+                    };
+                    order2(0, 1);
+                    order2(2, 3);
+                    order2(0, 2);
+                    order2(1, 3);
+                    order2(1, 2);
+                    // the slot's byte: unit offset from the node's child block, sign: a leaf
+                    const auto child = [&](uint32_t key_k) -> int {
+                        return (int)((uint32_t)__builtin_amdgcn_sbfe((int)q1.x, key_k, 8) & 0x8000007Fu) + (int)q0.w;
+                    };
+                    const auto entry = [&](uint32_t key_k) -> E {
+                        if constexpr (ANY) return child(key_k);
+                        else return (uint64_t)key_k << 32 | (uint32_t)child(key_k);
+                    };
+                    redo |= !st.push3(entry(key[3]), key[3] != 0xFFFFFFFFu, entry(key[2]), key[2] != 0xFFFFFFFFu,
+                                      entry(key[1]), key[1] != 0xFFFFFFFFu);
+                    node = key[0] != 0xFFFFFFFFu ? child(key[0]) : kSentinel;
+                }
+            } else if (at_leaf) {
+                const uint32_t rec = (uint32_t)leaf & 0x7FFFFFFFu;
+                const float4 *tp = reinterpret_cast<const float4 *>(a.wide + rec);
+                const float4 A = tp[0], B = tp[1], C = tp[2];
+                float t, u, v;
+                const bool end = fb(C.w) < 0;
+                leaf = end ? leaf2 : leaf + 3;
+                leaf2 = end ? 0 : leaf2;
+                if (tri_test<TRI>(A, B, C, ox, oy, oz, dx, dy, dz, tmin, ANY ? hit_t : bf(cull), &t, &u, &v)) {
+                    if (ANY) {
+                        const RayTerms r{idirx, idiry, idirz, ox * idirx, oy * idiry, oz * idirz, tmin};
+                        if (t < hit_t && in_leaf(a, fb(B.w), r, hit_t)) {
+                            hit_rec = 0;
+                            redo = false;
+                            st.clear();
+                            node = kSentinel;
+                            leaf = leaf2 = 0;
+                        }
+                    } else if (t < hit_t) {
+                        *reinterpret_cast<float4 *>(a.hits + rid) = make_float4(A.w, t, u, v);
+                        next_t = hit_t;
+                        hit_t = t;
+                        hit_rec = (int)rec;
+                        hit_place = fb(B.w);
+                        cull = fb(t * 1.0009765625f);
+                    } else if (t > hit_t || fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)hit_rec)->w) != fb(A.w)) {
+                        next_t = fminf(next_t, t);   // (at hit_t itself: unless it is the same triangle again)
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The two-child while-while loop: for scenes without a four-child tree (wide.hip) and for
+// the node-fetch probe. VARIANT 0 (exact): a lane leaves the node loop as soon as it holds
+// a leaf, the single-lane order; VARIANT 1 (speculative): lanes keep descending until no
+// lane of the wave is still searching for its first leaf (__any ballot, :192-203); results
+// can differ only where a triangle lies on a box boundary within rounding of the current
+// hit distance.
+// REC (closest hit only; the probe): 1 counts each ray's node visits, triangle tests and
+// leaf visits; 2 records at every node visit the slab test's outcome as a 4-bit code (bit
+// 0: child 0 entered, bit 1: child 1 entered, bit 2: both, child 1 first); 3 replays: the
+// same loop, stack, leaf postponement, ballots and refills, every node and triangle record
+// fetched, but each node's outcome read from the record instead of computed and no
+// triangle arithmetic.
 template <int VARIANT, bool ANY, int S, int TRI, int REC = 0>
 __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
     static_assert(REC == 0 || !ANY, "fetch recording follows the closest-hit loop");
@@ -107,15 +581,7 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
         if (a.reset0) *a.reset0 = 0;
         if (a.reset1) *a.reset1 = 0;
     }
-    // Persistent waves (Aila & Laine's persistent threads with ray replacement):
-    // the grid holds about as many waves as the chip keeps resident, and wave w of W
-    // owns the 64-ray groups w, w + W, w + 2W, ... in that order, so that all waves
-    // sweep the ray range together (the rays in flight at any moment lie in a window
-    // of about 2W groups, as with one block per group, which keeps coherent rays'
-    // nodes in cache). A lane whose ray is done writes its result and takes the next
-    // ray of its wave's sequence (ballot and prefix count, no atomics): the lanes
-    // stay busy until the sequence runs out, instead of idling behind the wave's
-    // longest ray. Each ray's traversal is the same as with one ray per lane.
+    // the launch form of k_trace_wide
     const int64_t groups = (n + 63) >> 6;
     const int64_t waves_all = (int64_t)gridDim.x * (blockDim.x >> 6);
     const int64_t waves = max((int64_t)1, min(waves_all, groups));
@@ -160,10 +626,6 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
             } else if (ANY) {
                 a.flags[rid] = hit_id != -1 ? 1 : 0;
             } else {
-                if (hit_id == -1) {
-                    hit_u = 0.0f;
-                    hit_v = 0.0f;
-                }
                 *reinterpret_cast<float4 *>(a.hits + rid) = make_float4(bf(hit_id), hit_t, hit_u, hit_v);
             }
             rid = -1;
@@ -198,7 +660,7 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
                 st.sp = 0;
                 st.off = 0;
                 leaf_addr = 0;
-                node_addr = a.num_nodes > 0 ? (a.ray_root ? a.ray_root[rid] : 0) : kSentinel;
+                node_addr = a.num_nodes > 0 ? (a.roots ? a.roots[a.ray_root ? a.ray_root[rid] : 0] : 0) : kSentinel;
                 hit_t = r1.w;
                 hit_u = 0.0f;
                 hit_v = 0.0f;
@@ -249,26 +711,10 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
                        (__float_as_uint(nz.x) ^ __float_as_uint(nz.y) ^ __float_as_uint(nz.z) ^ __float_as_uint(nz.w));
             } else {
 
-            const float c0lox = n0xy.x * idirx - oodx;
-            const float c0hix = n0xy.y * idirx - oodx;
-            const float c0loy = n0xy.z * idiry - oody;
-            const float c0hiy = n0xy.w * idiry - oody;
-            const float c0loz = nz.x * idirz - oodz;
-            const float c0hiz = nz.y * idirz - oodz;
-            const float c1loz = nz.z * idirz - oodz;
-            const float c1hiz = nz.w * idirz - oodz;
-            const float c0min = span_begin(c0lox, c0hix, c0loy, c0hiy, c0loz, c0hiz, tmin);
-            const float c0max = span_end(c0lox, c0hix, c0loy, c0hiy, c0loz, c0hiz, hit_t);
-            const float c1lox = n1xy.x * idirx - oodx;
-            const float c1hix = n1xy.y * idirx - oodx;
-            const float c1loy = n1xy.z * idiry - oody;
-            const float c1hiy = n1xy.w * idiry - oody;
-            const float c1min = span_begin(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, tmin);
-            const float c1max = span_end(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, hit_t);
-
-            const float ray_tmax = 1e20f;
-            t0 = (c0min <= c0max) && (c0min >= tmin) && (c0min <= ray_tmax);
-            t1 = (c1min <= c1max) && (c1min >= tmin) && (c1min <= ray_tmax);
+            const RayTerms r{idirx, idiry, idirz, oodx, oody, oodz, tmin};
+            float c0min, c1min;
+            t0 = slab(n0xy, nz.x, nz.y, r, hit_t, &c0min);
+            t1 = slab(n1xy, nz.z, nz.w, r, hit_t, &c1min);
             c1_first = c1min < c0min;
             if (REC == 2) {
                 const uint32_t code = (t0 ? 1u : 0u) | (t1 ? 2u : 0u) | ((t0 && t1 && c1_first) ? 4u : 0u);
@@ -329,45 +775,15 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
                     ++tri;
                     continue;
                 }
-                // Möller–Trumbore, IntersectKernel.cuh:230-254 (edges precomputed: same bits)
-                const float tvx = ox - A.x, tvy = oy - A.y, tvz = oz - A.z;
-                const float pvx = dy * C.z - dz * C.y;
-                const float pvy = dz * C.x - dx * C.z;
-                const float pvz = dx * C.y - dy * C.x;
-                const float det = B.x * pvx + B.y * pvy + B.z * pvz;
-                const float inv = 1.0f / det;
-                const float u = (tvx * pvx + tvy * pvy + tvz * pvz) * inv;
-                const float qvx = tvy * B.z - tvz * B.y;
-                const float qvy = tvz * B.x - tvx * B.z;
-                const float qvz = tvx * B.y - tvy * B.x;
-                const float v = (dx * qvx + dy * qvy + dz * qvz) * inv;
-                bool ok;
-                if (TRI == kTriReference) {
-                    const float EPS = 0.00001f;
-                    if (det > EPS) {
-                        ok = !(u < 0.0f || u > 1.0f) && !(v < 0.0f || (u + v) > 1.0f);
-                    } else if (det < -EPS) {
-                        // the reference's back-face bounds (IntersectKernel.cuh:248-250)
-                        // have their comparisons reversed: u > 0 || u < 1 always holds,
-                        // so back faces are never accepted; kept as written
-                        ok = !(u > 0.0f || u < 1.0f) && !(v > 0.0f || (u + v) < 1.0f);
-                    } else {
-                        ok = false;
-                    }
-                } else {
-                    ok = det != 0.0f && u >= 0.0f && u <= 1.0f && v >= 0.0f && (u + v) <= 1.0f;
-                }
-                if (ok) {
-                    const float t = (C.x * qvx + C.y * qvy + C.z * qvz) * inv;
-                    if (tmin < t && t < hit_t) {
-                        hit_t = t;
-                        hit_u = u;
-                        hit_v = v;
-                        hit_id = fb(A.w);
-                        if (ANY) {
-                            node_addr = kSentinel;
-                            break;
-                        }
+                float t, u, v;
+                if (tri_test<TRI>(A, B, C, ox, oy, oz, dx, dy, dz, tmin, hit_t, &t, &u, &v) && t < hit_t) {
+                    hit_t = t;
+                    hit_u = u;
+                    hit_v = v;
+                    hit_id = fb(A.w);
+                    if (ANY) {
+                        node_addr = kSentinel;
+                        break;
                     }
                 }
                 if (fb(C.w) != 0) break;
@@ -399,6 +815,19 @@ hipError_t launch_k(K kernel, const TraceArgs &a, bool persistent, int block, si
     return hipGetLastError();
 }
 
+template <bool ANY, int TRI>
+hipError_t launch_wide(const TraceArgs &a, bool persistent, int S, int block, int num_cus, hipStream_t s) {
+    // S entries for any-hit launches (4 bytes each), 3/4 S for closest-hit ones (8 bytes)
+    const size_t lds = (ANY ? (size_t)S * 4 : (size_t)S * 6) * block;
+    switch (S) {
+        case 8: return launch_k(k_trace_wide<ANY, ANY ? 8 : 6, TRI>, a, persistent, block, lds, num_cus, s);
+        case 16: return launch_k(k_trace_wide<ANY, ANY ? 16 : 12, TRI>, a, persistent, block, lds, num_cus, s);
+        case 24: return launch_k(k_trace_wide<ANY, ANY ? 24 : 18, TRI>, a, persistent, block, lds, num_cus, s);
+        case 32: return launch_k(k_trace_wide<ANY, ANY ? 32 : 24, TRI>, a, persistent, block, lds, num_cus, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 template <int V, bool ANY, int TRI>
 hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int num_cus, hipStream_t s) {
     const size_t lds = (size_t)S * block * sizeof(int);
@@ -411,15 +840,13 @@ hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int n
     }
 }
 
-template <int TRI>
-hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, bool any, int S, int block, int num_cus,
-                    hipStream_t s) {
-    if (variant == 0)
-        return any ? launch_s<0, true, TRI>(a, persistent, S, block, num_cus, s)
-                   : launch_s<0, false, TRI>(a, persistent, S, block, num_cus, s);
-    if (variant == 1)
-        return any ? launch_s<1, true, TRI>(a, persistent, S, block, num_cus, s)
-                   : launch_s<1, false, TRI>(a, persistent, S, block, num_cus, s);
+// The four-child walk where the scene has that tree (wide.hip builds it where it pays),
+// the two-child loop of the asked variant elsewhere.
+template <bool ANY, int TRI>
+hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int block, int num_cus, hipStream_t s) {
+    if (a.wide) return launch_wide<ANY, TRI>(a, persistent, S, block, num_cus, s);
+    if (variant == 0) return launch_s<0, ANY, TRI>(a, persistent, S, block, num_cus, s);
+    if (variant == 1) return launch_s<1, ANY, TRI>(a, persistent, S, block, num_cus, s);
     return hipErrorInvalidValue;
 }
 
@@ -445,15 +872,31 @@ hipError_t launch_trace(const TraceArgs &a, int variant, bool any, int lds_stack
                         int refill, int num_cus, hipStream_t s, int tri_mode) {
     if (a.n <= 0) return hipSuccess;
     if (block < 64 || block > 256 || block % 64 != 0) return hipErrorInvalidValue;
-    if ((a.n + block - 1) / block > 0x7FFFFFFF) return hipErrorInvalidValue;
     TraceArgs b = a;
     b.xcd_order = xcd_order ? 1 : 0;
     // refill 0: one wave per 64-ray group; 1..64: persistent waves with that threshold
     const bool persistent = refill > 0;
     b.refill = persistent ? (refill > 64 ? 64 : refill) : 64;
-    if (tri_mode == kTriReference) return launch_v<kTriReference>(b, persistent, variant, any, lds_stack, block, num_cus, s);
-    if (tri_mode == kTriTwoSided) return launch_v<kTriTwoSided>(b, persistent, variant, any, lds_stack, block, num_cus, s);
-    return hipErrorInvalidValue;
+    // ray indices are 32-bit in the kernel: more rays go in several launches (a device-side
+    // count or an order comes with fewer)
+    constexpr int64_t kPart = (int64_t)1 << 30;
+    if (a.n > kPart && (a.n_dev || a.order)) return hipErrorInvalidValue;
+    for (int64_t at = 0; at < a.n; at += kPart) {
+        b.n = std::min(kPart, a.n - at);
+        b.rays = a.rays + at;
+        if (a.hits) b.hits = a.hits + at;
+        if (a.flags) b.flags = a.flags + at;
+        if (a.ray_root) b.ray_root = a.ray_root + at;
+        hipError_t e = hipErrorInvalidValue;
+        if (tri_mode == kTriReference)
+            e = any ? launch_v<true, kTriReference>(b, persistent, variant, lds_stack, block, num_cus, s)
+                    : launch_v<false, kTriReference>(b, persistent, variant, lds_stack, block, num_cus, s);
+        else if (tri_mode == kTriTwoSided)
+            e = any ? launch_v<true, kTriTwoSided>(b, persistent, variant, lds_stack, block, num_cus, s)
+                    : launch_v<false, kTriTwoSided>(b, persistent, variant, lds_stack, block, num_cus, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace tt

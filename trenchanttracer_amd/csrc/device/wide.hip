@@ -1,0 +1,444 @@
+// The four-child tree k_trace_wide walks, built on the GPU from the two-child SBVH when a
+// scene is created.
+//
+// One array of 48-byte records (three 16-byte units), nodes and triangles alike; a
+// reference is a unit index below 2^30, with the sign bit set for a leaf. The scenes'
+// roots come first; a node's children lie together, inner nodes first, then the leaves'
+// triangle records. The walk is bound by VALU issue and by vector memory lane loads, so a
+// node is as few loads as four boxes and their children fit in, in the form that decodes
+// with the fewest operations:
+//   unit 0: origin x, y, z (floats), first unit of the child block
+//   unit 1: per slot a byte {leaf, unit offset in the block}; plane scales' exponents (x, y,
+//           z as signed bytes); x low planes (one byte per slot), x high planes
+//   unit 2: y low, y high, z low, z high planes
+// A plane is origin + byte * 2^exponent, rounded outwards. Slots hold the inner children,
+// then the leaves by rising triangle count (which keeps the offsets small), then empty
+// boxes. An empty box that the rounding allowance lets a ray enter leads to a leaf of the
+// node once more, or, where it has none, to a record no ray hits: never to a node.
+// Children: starting from a two-child node's two, the inner child with the largest box is
+// replaced by its own two while they fit (simulated on 1M-triangle soup: 24.2 visits of 3
+// loads per incoherent ray against 50.6 of 4; eight children with 80-byte nodes: 16.7
+// visits of 5). Triangle records are copied so that a node's leaves lie together; the
+// second word's w is the leaf's place in the two-child tree (node * 2 + child), the third's
+// the next record of the same triangle (a ring over its leaves), negative at a leaf's end.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../host/tt_host.h"
+#include "dev_common.h"
+#include "scene_dev.h"
+
+namespace tt {
+namespace {
+
+constexpr int kMaxOffset = 42;   // largest record offset of a slot (126 units)
+constexpr int32_t kRingEnd = 0x7FFFFFFF;   // no unit index
+
+struct WideBuild {
+    const float4 *nodes;
+    const float4 *tris;
+    const int32_t *roots;   // two-child roots of the scenes
+    int32_t nroots;
+    uint4 *wide;            // [3 * record]
+    // breadth-first list of the nodes: record, and place in the two-child tree (node * 2 +
+    // child; roots: unused)
+    int2 *list;
+    int32_t *last_of;       // [triangle id]: first unit of its record linked last, or -1
+    int32_t ids;            // triangle ids below this have a ring; others stand alone
+    int32_t *state;         // [0] nodes listed, [1] records allocated, [2] set: the tree does not fit
+    int32_t node_cap, rec_cap;
+};
+
+struct Child {
+    float lo[3], hi[3];
+    int32_t ref;      // two-child index: node, or ~first record
+    int32_t place;    // node * 2 + child
+    int32_t count;    // triangle records of a leaf (0: inner child)
+    int32_t ref2, count2, place2;   // a second leaf merged into the slot (count2 0: none)
+};
+
+__device__ void box_of(const float4 *nodes, int32_t node, int c, Child &k) {
+    const float4 xy = nodes[(int64_t)node * 4 + c];
+    const float4 z = nodes[(int64_t)node * 4 + 2];
+    k.lo[0] = xy.x;
+    k.hi[0] = xy.y;
+    k.lo[1] = xy.z;
+    k.hi[1] = xy.w;
+    k.lo[2] = c ? z.z : z.x;
+    k.hi[2] = c ? z.w : z.y;
+}
+
+__device__ float half_area(const Child &k) {
+    const float x = k.hi[0] - k.lo[0], y = k.hi[1] - k.lo[1], z = k.hi[2] - k.lo[2];
+    return x * y + y * z + z * x;
+}
+
+// Appends the children of a two-child node to out; a leaf without triangles (one record
+// with zero edges) is left out. False where a box is not finite, is inverted, or leaves
+// the node's own (in): such trees keep the two-child walk alone.
+__device__ bool add_children(const WideBuild &b, int32_t node, const Child *in, Child *out, int &n) {
+    const int4 ch = reinterpret_cast<const int4 *>(b.nodes)[(int64_t)node * 4 + 3];
+    for (int c = 0; c < 2; ++c) {
+        Child k{};
+        k.ref = c ? ch.y : ch.x;
+        k.place = node * 2 + c;
+        if (k.ref < 0) {
+            const float4 *t = b.tris + (int64_t)~k.ref * 3;
+            while (__float_as_int(t[3 * k.count + 2].w) == 0) ++k.count;
+            ++k.count;
+            if (k.count == 1 && t[1].x == 0.0f && t[1].y == 0.0f && t[1].z == 0.0f && t[2].x == 0.0f && t[2].y == 0.0f &&
+                t[2].z == 0.0f)
+                continue;
+        }
+        box_of(b.nodes, node, c, k);
+        for (int q = 0; q < 3; ++q) {
+            if (!(fabsf(k.lo[q]) < 0x1p60f && fabsf(k.hi[q]) < 0x1p60f && k.lo[q] <= k.hi[q])) return false;
+            if (in && !(in->lo[q] <= k.lo[q] && k.hi[q] <= in->hi[q])) return false;
+        }
+        out[n++] = k;
+    }
+    return true;
+}
+
+// Whether the leaves among c[0, n) can be addressed: the inner children and all leaves but
+// the largest lie before it.
+__device__ bool leaves_fit(const Child *c, int n) {
+    int64_t before = 0, most = 0;
+    for (int k = 0; k < n; ++k) {
+        before += c[k].count ? c[k].count : 1;
+        most = max(most, (int64_t)c[k].count);
+    }
+    return before - most <= kMaxOffset;
+}
+
+__device__ int wave_scan(int v, int *total) {   // exclusive sum over the wave's lanes
+    int s = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(s, o);
+        if ((int)__lane_id() >= o) s += y;
+    }
+    *total = __shfl(s, 63);
+    return s - v;
+}
+
+__device__ void copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_t place, int32_t at, bool last) {
+    const float4 *t = b.tris + (int64_t)~ref * 3;
+    float4 *to = reinterpret_cast<float4 *>(b.wide) + (int64_t)at * 3;
+    for (int i = 0; i < count; ++i) {
+        float4 e1 = t[3 * i + 1], e2 = t[3 * i + 2];
+        const int32_t id = __float_as_int(t[3 * i].w);
+        // the record before this one in the ring; the first closes it (k_wide_rings)
+        int32_t link = id >= 0 && id < b.ids ? atomicExch(&b.last_of[id], 3 * (at + i)) : 3 * (at + i);
+        if (link < 0) link = kRingEnd;
+        e1.w = __int_as_float(place);
+        e2.w = __int_as_float(link | (last && i + 1 == count ? (int32_t)0x80000000 : 0));
+        to[3 * i] = t[3 * i];
+        to[3 * i + 1] = e1;
+        to[3 * i + 2] = e2;
+    }
+}
+
+// Closes the rings: the record linked first (it holds kRingEnd) points to the one linked
+// last. One thread per triangle id, which follows its ring to that record.
+__global__ __launch_bounds__(256) void k_wide_rings(WideBuild b) {
+    const int32_t id = blockIdx.x * 256 + threadIdx.x;
+    if (id >= b.ids || b.last_of[id] < 0) return;
+    const int32_t last = b.last_of[id];
+    for (int32_t at = last;;) {
+        int32_t *link = reinterpret_cast<int32_t *>(b.wide + at + 2) + 3;
+        const int32_t v = *link;
+        if ((v & 0x7FFFFFFF) == kRingEnd) {
+            *link = last | (v & (int32_t)0x80000000);
+            return;
+        }
+        at = v & 0x7FFFFFFF;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_wide_clear(int32_t *p, int32_t n) {
+    const int32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = -1;
+}
+
+// One level of the tree: nodes [first, first + count) of the list, one thread each. A
+// wave's child blocks come from one atomic add on the records, its inner children are
+// listed (the next level) from another.
+__global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, int32_t count) {
+    const int32_t i = first + (int32_t)(blockIdx.x * 64 + threadIdx.x);
+    const bool live = i < first + count;
+    int32_t self_rec = 0;
+    Child c[4];
+    int n = 0;
+    bool bad = false;
+    if (live) {
+        if (i < b.nroots) {
+            self_rec = i;
+            bad = !add_children(b, b.roots[i], nullptr, c, n);
+        } else {
+            self_rec = b.list[i].x;
+            const int32_t p = b.list[i].y;
+            Child self{};
+            box_of(b.nodes, p >> 1, p & 1, self);
+            const int4 ch = reinterpret_cast<const int4 *>(b.nodes)[(int64_t)(p >> 1) * 4 + 3];
+            bad = !add_children(b, (p & 1) ? ch.y : ch.x, &self, c, n);
+        }
+        if (!bad && n == 2 && !leaves_fit(c, n)) {
+            // two large leaves: one slot for both
+            c[0].ref2 = c[1].ref;
+            c[0].count2 = c[1].count;
+            c[0].place2 = c[1].place;
+            for (int q = 0; q < 3; ++q) {
+                c[0].lo[q] = fminf(c[0].lo[q], c[1].lo[q]);
+                c[0].hi[q] = fmaxf(c[0].hi[q], c[1].hi[q]);
+            }
+            n = 1;
+        }
+        bool shut[4] = {false, false, false, false};   // opening it would not fit
+        while (!bad && n < 4) {
+            int best = -1;
+            float area = -1.0f;
+            for (int k = 0; k < n; ++k)
+                if (c[k].count == 0 && !shut[k] && half_area(c[k]) > area) {
+                    area = half_area(c[k]);
+                    best = k;
+                }
+            if (best < 0) break;
+            Child two[2], trial[4];
+            int m = 0, t = 0;
+            bad = !add_children(b, c[best].ref, &c[best], two, m);
+            for (int k = 0; k < n; ++k)
+                if (k != best) trial[t++] = c[k];
+            for (int k = 0; k < m; ++k) trial[t++] = two[k];
+            if (bad) break;
+            if (!leaves_fit(trial, t)) {
+                shut[best] = true;
+                continue;
+            }
+            // the slots moved: whatever was shut is tried again (it still does not fit)
+            n = t;
+            for (int k = 0; k < n; ++k) {
+                c[k] = trial[k];
+                shut[k] = false;
+            }
+        }
+        // inner children, then leaves by rising count (insertion sort)
+        for (int k = 1; k < n; ++k)
+            for (int j = k; j > 0 && c[j].count < c[j - 1].count; --j) {
+                const Child x = c[j];
+                c[j] = c[j - 1];
+                c[j - 1] = x;
+            }
+    }
+    int inner = 0;
+    int64_t records = 0;
+    if (live && !bad)
+        for (int k = 0; k < n; ++k) {
+            inner += c[k].count == 0;
+            records += c[k].count ? (int64_t)c[k].count + c[k].count2 : 1;
+        }
+    // the empty slots' leaf: the node's first, or a record of its own
+    const bool no_leaf = live && !bad && n < 4 && inner == n;
+    if (no_leaf) ++records;
+    if (records > b.rec_cap) bad = true;
+    int nodes_all = 0, recs_all = 0;
+    int node0 = wave_scan(bad ? 0 : inner, &nodes_all);
+    int rec0 = wave_scan(bad ? 0 : (int)records, &recs_all);
+    int at[2] = {0, 0};
+    if (__lane_id() == 63) {
+        at[0] = atomicAdd(&b.state[0], nodes_all);
+        at[1] = atomicAdd(&b.state[1], recs_all);
+    }
+    node0 += __shfl(at[0], 63);
+    rec0 += __shfl(at[1], 63);
+    if (!live) return;
+    if (node0 < 0 || rec0 < 0 || (int64_t)node0 + inner > b.node_cap || (int64_t)rec0 + records > b.rec_cap) bad = true;
+    if (bad) {
+        b.state[2] = 1;
+        return;
+    }
+    // the box of all children, the scales and the planes
+    float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < n; ++k)
+        for (int q = 0; q < 3; ++q) {
+            lo[q] = k ? fminf(lo[q], c[k].lo[q]) : c[k].lo[q];
+            hi[q] = k ? fmaxf(hi[q], c[k].hi[q]) : c[k].hi[q];
+        }
+    uint32_t code[3], planes[3][2] = {{0xFFFFFFFFu, 0u}, {0xFFFFFFFFu, 0u}, {0xFFFFFFFFu, 0u}};
+    for (int q = 0; q < 3; ++q) {
+        // the smallest power of two with 255 steps over the extent
+        int e = -126;
+        const double step = ((double)hi[q] - (double)lo[q]) / 255.0;
+        if (step > 0.0) {
+            const double m = frexp(step, &e);
+            if (m == 0.5) --e;
+            e = max(e, -126);
+        }
+        code[q] = (uint32_t)e & 255u;
+        const double inv = ldexp(1.0, -e);
+        for (int k = 0; k < n; ++k) {
+            const uint32_t l = (uint32_t)floor(((double)c[k].lo[q] - (double)lo[q]) * inv);
+            const uint32_t h = (uint32_t)ceil(((double)c[k].hi[q] - (double)lo[q]) * inv);
+            if (l > 255u || h > 255u) {
+                b.state[2] = 1;
+                return;
+            }
+            planes[q][0] = (planes[q][0] & ~(255u << (8 * k))) | l << (8 * k);
+            planes[q][1] |= h << (8 * k);
+        }
+    }
+    uint32_t offsets = 0;
+    int32_t off = 0;
+    for (int k = 0; k < n; ++k) {
+        if (c[k].count == 0) {
+            b.list[node0 + k] = make_int2(rec0 + k, c[k].place);
+            offsets |= (uint32_t)(3 * off) << (8 * k);
+            ++off;
+            continue;
+        }
+        offsets |= (uint32_t)(128 | 3 * off) << (8 * k);
+        copy_leaf(b, c[k].ref, c[k].count, c[k].place, rec0 + off, c[k].count2 == 0);
+        if (c[k].count2) copy_leaf(b, c[k].ref2, c[k].count2, c[k].place2, rec0 + off + c[k].count, true);
+        off += c[k].count + c[k].count2;
+    }
+    if (no_leaf) {
+        // no edges (never accepted), no triangle, its own ring, the end of its leaf
+        float4 *to = reinterpret_cast<float4 *>(b.wide) + ((int64_t)rec0 + off) * 3;
+        to[0] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
+        to[1] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+        to[2] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(3 * (rec0 + off) | (int32_t)0x80000000));
+    }
+    for (int k = n; k < 4; ++k) offsets |= (uint32_t)(128 | 3 * inner) << (8 * k);
+    uint4 *w = b.wide + (int64_t)self_rec * 3;
+    w[0] = make_uint4(__float_as_uint(lo[0]), __float_as_uint(lo[1]), __float_as_uint(lo[2]),
+                      3u * (uint32_t)rec0);
+    w[1] = make_uint4(offsets, code[0] | code[1] << 8 | code[2] << 16, planes[0][0], planes[0][1]);
+    w[2] = make_uint4(planes[1][0], planes[1][1], planes[2][0], planes[2][1]);
+}
+
+// Whether a random line through the tree's root box is expected to cost more than `limit`
+// box pairs and triangle tests (the surface-area sum of BVHNode::computeSubtreeProbabilities:
+// 2 per inner node, 1 per triangle, each weighted by its box's share of the root's area).
+// Boxes below 1/256 of the root's area are left out, so the walk ends within 256 x limit nodes.
+bool costs_more_than(const std::vector<int32_t> &nodes, int32_t root, double limit) {
+    double sum = 2.0, root_area = -1.0;
+    std::vector<int32_t> stack{root};
+    while (!stack.empty() && sum <= limit) {
+        const int32_t *w = &nodes[(size_t)stack.back() * 16];
+        stack.pop_back();
+        float f[12];
+        std::memcpy(f, w, sizeof(f));
+        double area[2];
+        for (int c = 0; c < 2; ++c) {
+            const double x = (double)f[4 * c + 1] - f[4 * c], y = (double)f[4 * c + 3] - f[4 * c + 2],
+                         z = (double)f[9 + 2 * c] - f[8 + 2 * c];
+            area[c] = x >= 0.0 && y >= 0.0 && z >= 0.0 ? x * y + y * z + z * x : 0.0;
+        }
+        if (root_area < 0.0) {
+            const double x = std::max(f[1], f[5]) - (double)std::min(f[0], f[4]),
+                         y = std::max(f[3], f[7]) - (double)std::min(f[2], f[6]),
+                         z = std::max(f[9], f[11]) - (double)std::min(f[8], f[10]);
+            root_area = x * y + y * z + z * x;
+            if (!(root_area > 0.0 && root_area < INFINITY)) return false;
+        }
+        for (int c = 0; c < 2; ++c) {
+            const double p = area[c] / root_area;
+            sum += p * (w[12 + c] < 0 ? w[14 + c] : 2);
+            if (w[12 + c] >= 0 && p >= 1.0 / 256) stack.push_back(w[12 + c]);
+        }
+    }
+    return sum > limit;
+}
+
+}  // namespace
+
+// Builds s->wide for the scene's uploaded two-child tree; roots: the scenes' root nodes
+// (node 0 alone for a single scene). Leaves it null where the tree does not fit the format,
+// memory is short, or rays are expected to be short: every ray then walks the two-child
+// tree. The four-child walk has more to do per ray (setting up, checking its winner's leaf)
+// and holds 6 waves per SIMD instead of 8; per node and triangle it is faster. Measured, by
+// expected cost (closest hit, us, two-child / four-child): Cornell box with a 5120-triangle
+// sphere 4.0, 64-spp reference render 2573 / 2703; closed room of 20 triangles 15, 64-spp
+// render 2166 / 2341; soups of 524288 rays: 30 triangles 11, 38 / 38; 100 triangles 24,
+// 79 / 68; 300 triangles 37, 130 / 97; 10000 triangles 155, 341 / 242.
+tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const std::vector<int32_t> &roots) {
+    // nodes at most as many as the two-child tree has; units below 2^30
+    const int64_t recs = s->num_nodes + s->num_tris;
+    if (s->num_nodes == 0 || recs >= (1 << 30) / 3) return TT_OK;
+    constexpr double kShort = 20.0;
+    if (std::none_of(roots.begin(), roots.end(), [&](int32_t r) { return costs_more_than(dev_nodes, r, kShort); }))
+        return TT_OK;
+    // the largest coordinate of the scenes' boxes (a plane can lie one step past its box)
+    double bound = 0.0;
+    for (const int32_t r : roots) {
+        float w[12];
+        std::memcpy(w, &dev_nodes[(size_t)r * 16], sizeof(w));
+        const int lo_at[3] = {0, 2, 8};
+        for (int q = 0; q < 3; ++q) {
+            const float *a = w + lo_at[q], *c = w + lo_at[q] + (q == 2 ? 2 : 4);
+            for (const float *p : {a, c})
+                if (p[0] <= p[1])   // a leaf without triangles has an inverted box
+                    bound = std::max(bound, std::max(std::fabs((double)p[0]), std::fabs((double)p[1])));
+        }
+    }
+    if (!(bound < 0x1p60)) return TT_OK;
+    void *mem = nullptr, *tmp = nullptr;
+    const size_t bytes = (size_t)recs * 48;
+    // triangle ids (0 .. max(id)): those of the scene's mesh, or of as many records as there are
+    const int32_t ids = (int32_t)std::max<int64_t>(s->num_orig_tris, s->num_tris);
+    const size_t list_bytes = (size_t)s->num_nodes * 8, root_bytes = roots.size() * 4;
+    if (hipMalloc(&mem, bytes) != hipSuccess ||
+        hipMalloc(&tmp, 16 + list_bytes + root_bytes + (size_t)ids * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        if (mem) hipFree(mem);
+        return TT_OK;
+    }
+    WideBuild b{};
+    b.nodes = reinterpret_cast<const float4 *>(s->nodes);
+    b.tris = reinterpret_cast<const float4 *>(s->tris);
+    b.wide = static_cast<uint4 *>(mem);
+    b.state = static_cast<int32_t *>(tmp);
+    b.list = reinterpret_cast<int2 *>(b.state + 4);
+    int32_t *d_roots = b.state + 4 + 2 * s->num_nodes;
+    b.roots = d_roots;
+    b.nroots = (int32_t)roots.size();
+    b.last_of = d_roots + roots.size();
+    b.ids = ids;
+    b.node_cap = (int32_t)s->num_nodes;
+    b.rec_cap = (int32_t)recs;
+    int32_t state[4] = {b.nroots, b.nroots, 0, 0};
+    hipStream_t hs = s->ctx->stream;
+    hipError_t err = hipMemcpyAsync(b.state, state, sizeof(state), hipMemcpyHostToDevice, hs);
+    if (err == hipSuccess) err = hipMemcpyAsync(d_roots, roots.data(), root_bytes, hipMemcpyHostToDevice, hs);
+    if (err == hipSuccess && ids > 0) {
+        hipLaunchKernelGGL(k_wide_clear, dim3((unsigned)((ids + 255) / 256)), dim3(256), 0, hs, b.last_of, ids);
+        err = hipGetLastError();
+    }
+    for (int32_t first = 0; err == hipSuccess && first < state[0] && state[2] == 0;) {
+        const int32_t count = state[0] - first;
+        hipLaunchKernelGGL(k_wide_level, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, hs, b, first, count);
+        err = hipGetLastError();
+        first += count;
+        if (err == hipSuccess) err = hipMemcpyAsync(state, b.state, sizeof(state), hipMemcpyDeviceToHost, hs);
+        if (err == hipSuccess) err = hipStreamSynchronize(hs);
+    }
+    if (err == hipSuccess && state[2] == 0 && ids > 0) {
+        hipLaunchKernelGGL(k_wide_rings, dim3((unsigned)((ids + 255) / 256)), dim3(256), 0, hs, b);
+        err = hipGetLastError();
+    }
+    const hipError_t end = hipStreamSynchronize(hs);
+    if (err == hipSuccess) err = end;
+    hipFree(tmp);
+    if (err != hipSuccess || state[2]) {
+        hipFree(mem);
+        return err == hipSuccess ? TT_OK : fail(TT_ERR_DEVICE, std::string("scene tree: ") + hipGetErrorString(err));
+    }
+    s->wide = mem;
+    s->wide_bound = (float)(bound * (1.0 + 4.0 / 255.0)) * 1.0001f;
+    s->bytes += bytes;
+    return TT_OK;
+}
+
+}  // namespace tt
