@@ -269,11 +269,12 @@ tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double 
  * (Aila-Laine postponed leaf + wave ballot). lds_stack: LDS stack entries of 4 bytes per
  * lane (8, 16, 24 or 32; a closest-hit entry of the four-child walk is 8 bytes, and 3/4 of
  * the number of them are kept in LDS); block: threads per block (64..256, multiple of 64).
- * refill: 0 (default) = one wave per 64-ray group; 1..64 = persistent waves: the
- * launch holds as many waves as the GPU keeps resident, wave w of W traces the
- * 64-ray groups w, w + W, ..., and a lane whose ray is done takes the wave's next ray
- * once at least `refill` of its 64 lanes are idle (keeps incoherent waves full; on
- * the 1M-soup traversal workload, half coherent rays, one wave per group is faster).
+ * refill: 0 (default) = the library's choice: sweeps over one part of the range after
+ * another, 4 64-ray groups per resident wave each (scenes that keep the two-child loop:
+ * one wave per group); 1..64 = persistent waves: the launch holds as many waves as the
+ * GPU keeps resident, wave w of W traces the 64-ray groups w, w + W, ..., and a lane whose
+ * ray is done takes the wave's next ray once at least `refill` of its 64 lanes are idle
+ * (keeps incoherent waves full; sweeps take rays at 32).
  * xcd_order: 0 = waves in launch order; 1 = blocks are renumbered so that each of the
  * 8 XCDs (which take blocks round-robin) holds one contiguous range of waves.
  * reorder: 0 (default) = rays are traced in the caller's order; 1 = the call first
@@ -302,8 +303,8 @@ typedef struct tt_trace_cfg {
 /* Closest hit for n rays (replaces intersect(ray, bvh, true),
  * include/geometry/IntersectKernel.cuh:78-296). rays / hits are DEVICE pointers; stream is a hipStream_t
  * (NULL = the context stream). Asynchronous: synchronise before reading hits.
- * cfg may be NULL: exact loop, 16 LDS entries, 128-thread blocks, one wave per 64-ray
- * group (trenchanttracer_amd.autotune.tune_trace picks a configuration per workload). */
+ * cfg may be NULL: exact loop, 16 LDS entries, 128-thread blocks, refill 0
+ * (trenchanttracer_amd.autotune.tune_trace picks a configuration per workload). */
 tt_status tt_trace_closest(tt_scene *s, const tt_ray *rays, int64_t n, tt_hit *hits,
                            const tt_trace_cfg *cfg, void *stream);
 /* Any hit (shadow rays; intersect(ray, bvh, false), IntersectKernel.cuh:265-269):

@@ -147,3 +147,29 @@ def test_four_child_walk_of_several_trees(tt, ctx):
         assert np.array_equal(one.view(np.int32), im.view(np.int32))
         s.close()
     batch.close()
+
+
+def test_sweeps_trace_every_ray_once(tt, ctx):
+    """refill 0 traces the range in parts; ray counts below, at and past one group per
+    resident wave and one part, ragged: the records of the persistent launch, and nothing
+    written past the end."""
+    mesh = tt.Mesh.soup(20000, seed=6)
+    scene = tt.DeviceScene(ctx, mesh, tt.BVH.build(mesh))
+    rays = tt.rays_incoherent(mesh, 3_000_017, seed=7)
+    d = tt.DeviceBuffer.from_array(ctx, rays)
+    h = tt.DeviceBuffer(ctx, (len(rays) + 64) * 16)
+
+    def trace(n, cfg):
+        h.upload(np.full((n + 64, 4), 7.0, np.float32))
+        scene.trace_closest(d, n, h, cfg)
+        ctx.sync()
+        return h.download((n + 64, 4), np.int32)
+    for n in (65_537, 327_681, 393_217, 700_001, 1_572_863, 1_572_865, 3_000_017):
+        print(f"sweeps: {n} rays", file=sys.stderr, flush=True)
+        for block in (64, 256):
+            got = trace(n, tt.trace_cfg(0, 16, block))
+            assert np.array_equal(got, trace(n, tt.trace_cfg(0, 16, block, refill=8)))
+            assert (got[n:].view(np.float32) == 7.0).all()
+    d.free()
+    h.free()
+    scene.close()

@@ -2,7 +2,7 @@
 
 Times short runs of candidate launch configurations on the actual workload and
 keeps the fastest: traversal loop variant x LDS stack entries x block size x
-launch form (one wave per 64-ray group, or persistent waves with lane refill) for
+launch form (sweeps, or persistent waves with lane refill) for
 `tune_trace`; paths in flight, hipGraph replay, traversal LDS stack, block size,
 refill and the pixel tile the path slots walk for `tune_render` (coordinate
 descent).
@@ -32,7 +32,7 @@ def _save(path, data):
 def tune_trace(ctx, scene, d_rays, n, d_hits, variants=(0, 1), lds=(8, 16, 24), blocks=(64, 128, 256),
                refills=(0, 16, 32), reorders=(0, 1), reps=3, exact_only=True, cache=None, key=None):
     """Fastest trace configuration for this scene and ray buffer: loop variant, LDS
-    stack depth, block size, launch form (refill 0: one wave per 64-ray group;
+    stack depth, block size, launch form (refill 0: sweeps over parts of the range;
     > 0: persistent waves that take new rays once that many lanes are idle) and ray
     order (reorder 1: traced in Morton order of the origins). With exact_only the
     speculative variant is not considered."""

@@ -311,22 +311,31 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
         if (a.reset0) *a.reset0 = 0;
         if (a.reset1) *a.reset1 = 0;
     }
-    // Persistent waves (Aila & Laine's persistent threads with ray replacement):
-    // the grid holds about as many waves as the chip keeps resident, and wave w of W
-    // owns the 64-ray groups w, w + W, w + 2W, ... in that order, so that all waves
-    // sweep the ray range together (the rays in flight at any moment lie in a window
-    // of about 2W groups, as with one block per group, which keeps coherent rays'
-    // nodes in cache). A lane whose ray is done writes its result and takes the next
-    // ray of its wave's sequence (ballot and prefix count, no atomics): the lanes
-    // stay busy until the sequence runs out, instead of idling behind the wave's
-    // longest ray. Each ray's traversal is the same as with one ray per lane. The wave's
-    // number is read from its first lane, so that everything uniform stays in scalar
-    // registers and the loops below branch on scalars.
+    // Launch forms. One wave per 64-ray group; persistent waves (Aila & Laine's persistent
+    // threads with ray replacement): the grid holds about as many waves as the chip keeps
+    // resident, and wave w of W owns the groups w, w + W, w + 2W, ... in that order, so that
+    // all waves sweep the ray range together (the rays in flight at any moment lie in a
+    // window of about 2W groups, as with one wave per group, which keeps coherent rays'
+    // nodes in cache); and sweeps: the same over one part of the range after another, W
+    // waves and a.sweep groups each per part, so that the waves cannot drift apart over a
+    // long range and the dispatcher evens out their loads. A lane whose ray is done takes
+    // the next ray of its wave's sequence (ballot and prefix count, no atomics): the lanes
+    // stay busy until the sequence runs out, instead of idling behind the wave's longest
+    // ray. Each ray's traversal is the same as with one ray per lane. The wave's number is
+    // read from its first lane, so that everything uniform stays in scalar registers and
+    // the loops below branch on scalars.
     const uint32_t groups = (n + 63u) >> 6;
-    const uint32_t waves = max(1u, min(gridDim.x * (blockDim.x >> 6), groups));
     const uint32_t w = vb * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
-    if (w >= waves) return;   // whole waves only: nothing below synchronises the block
-    const uint32_t total = ((groups - w + waves - 1u) / waves) * 64u;   // the wave's sequence positions
+    uint32_t waves = max(1u, min(gridDim.x * (blockDim.x >> 6), groups)), first = w, last = groups;
+    if (a.sweep) {
+        waves = (uint32_t)a.sweep_waves;
+        const uint32_t part = w / waves, size = waves * (uint32_t)a.sweep;
+        first = part * size + (w - part * waves);
+        last = min(groups, (part + 1u) * size);
+    }
+    // whole waves only: nothing below synchronises the block
+    if (first >= last || (!a.sweep && w >= waves)) return;
+    const uint32_t total = ((last - first + waves - 1u) / waves) * 64u;   // the wave's sequence positions
     const unsigned long long below = (1ull << lane) - 1ull;
 
     // one private array serves both walks
@@ -382,7 +391,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
         if (take && done) {
             const uint32_t q = cursor + (uint32_t)__popcll(m & below);
             if (q < total) {
-                const uint32_t r = ((q >> 6) * waves + w) * 64u + (q & 63u);
+                const uint32_t r = ((q >> 6) * waves + first) * 64u + (q & 63u);
                 if (r < n) rid = (int)(a.order ? a.order[r] : r);
             }
             if (rid >= 0) {
@@ -799,16 +808,28 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
 // instantiation at this block size and LDS), and for a known ray count no more
 // blocks than 64-ray groups. Otherwise one wave per 64-ray group (every wave's
 // sequence is its one group): the hardware dispatcher then balances the waves,
-// which wins where rays are coherent or the count is known.
+// which wins where rays are coherent or the count is known. With a.sweep (a known count)
+// the range is traced in parts of that many groups per resident wave; a range of at most
+// one group per wave is a launch of one wave per group.
 template <class K>
-hipError_t launch_k(K kernel, const TraceArgs &a, bool persistent, int block, size_t lds, int num_cus, hipStream_t s) {
+hipError_t launch_k(K kernel, TraceArgs a, bool persistent, int block, size_t lds, int num_cus, hipStream_t s) {
     int64_t grid = (a.n + block - 1) / block;
     if (persistent) {
         int per_cu = 0;
         hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds);
         if (e != hipSuccess) return e;
-        int64_t resident = (int64_t)std::max(1, per_cu) * std::max(1, num_cus);
-        grid = a.n_dev ? resident : std::min<int64_t>(resident, (a.n + 63) / 64);
+        const int64_t resident = (int64_t)std::max(1, per_cu) * std::max(1, num_cus);
+        const int64_t groups = (a.n + 63) / 64, waves = resident * (block / 64);
+        if (a.sweep && groups > waves) {
+            a.sweep_waves = (int32_t)waves;
+            const int64_t part = waves * a.sweep;
+            grid = (groups + part - 1) / part * resident;
+        } else if (a.sweep) {
+            a.sweep = 0;
+            a.refill = 64;
+        } else {
+            grid = a.n_dev ? resident : std::min<int64_t>(resident, groups);
+        }
     }
     grid = std::max<int64_t>(1, grid);
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(block), lds, s, a);
@@ -844,7 +865,21 @@ hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int n
 // the two-child loop of the asked variant elsewhere.
 template <bool ANY, int TRI>
 hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int block, int num_cus, hipStream_t s) {
-    if (a.wide) return launch_wide<ANY, TRI>(a, persistent, S, block, num_cus, s);
+    if (a.wide) {
+        // refill 0 and the count known here: sweeps of 4 groups per wave, taking rays at 32
+        // idle lanes. Against one wave per group and one persistent range (us): 1M shadow
+        // rays 556 / 386, with sweeps 389; 1.8M rays in 250k triangles 960 / 846, 846, its
+        // camera half 425 / 383, 385; 8.3M unsorted rays in 1M triangles 3915 / 4028, 3783.
+        // (2 groups: 470, 882, 3736; 8 groups: 386, 837, 3904.) A renderer's camera rays,
+        // many through one pixel, are the exception: 1080p at 64 samples 102.7 ms with one
+        // wave per group, 105.3 in sweeps, 110.1 persistent; their count is on the device.
+        TraceArgs b = a;
+        if (!persistent && !a.n_dev) {
+            b.sweep = 4;
+            b.refill = 32;
+        }
+        return launch_wide<ANY, TRI>(b, persistent || b.sweep, S, block, num_cus, s);
+    }
     if (variant == 0) return launch_s<0, ANY, TRI>(a, persistent, S, block, num_cus, s);
     if (variant == 1) return launch_s<1, ANY, TRI>(a, persistent, S, block, num_cus, s);
     return hipErrorInvalidValue;
