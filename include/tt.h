@@ -384,8 +384,8 @@ typedef struct tt_render_params {
                                  pass runs on one stream; otherwise path mode runs each bounce's
                                  next-event work on the context's second stream) */
     int32_t paths_in_flight;  /* target paths per pass, rounded to whole samples (0 = up to
-                                 2^27 paths, 256 B of state each, 488 B with a guide;
-                                 guided renders that train the network: about 8M) */
+                                 2^27 paths, 256 B of state each (272 B with several
+                                 scenes), 232 B more with a guide; guided renders that train the network: about 8M) */
     int32_t lds_stack;        /* traversal LDS stack entries per lane (0 = 16) */
     int32_t block;            /* traversal block size (0 = 64) */
     int32_t variant;          /* path-mode traversal loop: -1 speculative (default), 0 exact, 1 speculative */

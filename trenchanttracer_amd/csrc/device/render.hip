@@ -35,16 +35,16 @@ struct RenderState {
     int32_t cap = 0;
     tt_ray *rays[2] = {nullptr, nullptr};
     int32_t *path[2] = {nullptr, nullptr};
-    int32_t *root[2] = {nullptr, nullptr};   // scene of each queued ray
+    int32_t *root[2] = {nullptr, nullptr};   // several scenes: scene of each queued ray
     // next-event queues of even and odd bounces (a bounce's shadow work may still run
     // while the next bounce fills the other set)
     int32_t *sroot[2] = {nullptr, nullptr};
     int32_t *sample_dev = nullptr;            // first sample index of the current pass
     void *table = nullptr;                    // device SceneTable
     tt_hit *hits = nullptr;
-    // reference: mask | path: throughput, w = density of the last BSDF sample, or -1 when
-    // that sample was a specular (delta) one
-    float4 *thr = nullptr;
+    // reference: mask, by path id in [0] | path: throughput by queue slot (beside rays[k]),
+    // w = density of the last BSDF sample, or -1 when that sample was a specular (delta) one
+    float4 *thr[2] = {nullptr, nullptr};
     float4 *L = nullptr;         // reference: path radiance | path: x roulette weight, yzw radiance
     float4 *Lsh = nullptr;       // path: next-event radiance (xyz), added to L's at the end of the pass
     tt_ray *srays[2] = {nullptr, nullptr};     // next-event rays
@@ -56,6 +56,7 @@ struct RenderState {
     double *acc64 = nullptr;     // per pixel rgb (FP64 accumulation)
     int32_t acc64_cap = 0;
     int32_t pix_cap = 0;
+    bool roots = false;          // root and sroot are there
 };
 
 namespace tt {
@@ -253,13 +254,13 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a) {
     }
     f3 d = vnorm(vnorm(on_image - ap));
     a.rays[p] = {ap.x, ap.y, ap.z, a.tmin, d.x, d.y, d.z, 1e20f};
-    a.path[p] = p;
-    a.root[p] = sid;
-    // reference mode: mask and path radiance. Path mode starts every path from
+    if (a.root) a.root[p] = sid;
+    // reference mode: path id, mask and path radiance. Path mode starts every path from
     // throughput 1 and roulette weight 1, which its camera-bounce shading takes as
-    // constants (every generated path is in that bounce's queue), so nothing is
-    // written here.
+    // constants (every generated path is in that bounce's queue, path p in slot p), so
+    // nothing is written here.
     if (a.mode != TT_RENDER_PATH) {
+        a.path[p] = p;
         a.thr[p] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
         if (a.L) a.L[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
@@ -470,10 +471,12 @@ struct ShadeArgs {
     const int32_t *sample_dev;
     tt_ray *rays_in, *rays_out;
     int32_t *path_in, *path_out;
-    const int32_t *root_in;
-    int32_t *root_out, *sroot;
+    int32_t *root_out, *sroot;   // scenes of the queued rays (null: one scene)
     const tt_hit *hits;
-    float4 *thr, *L;
+    float4 *thr;                 // reference: by path id
+    const float4 *thr_in;        // path: by slot of rays_in
+    float4 *thr_out;
+    float4 *L;
     float4 *Lsh;       // zeroed for every path on the camera bounce
     int32_t *counts;
     int32_t cur, nxt;
@@ -522,10 +525,8 @@ __device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const in
     tt_ray nr{};
     if (i < n) {
         p = a.path_in[i];
-        root = a.root_in[i];
-        int sid_;
         int32_t x_, y_;
-        const int32_t local = pixel_of_slot(a.tab, path_slot(p, a.k), &sid_, &x_, &y_);
+        const int32_t local = pixel_of_slot(a.tab, path_slot(p, a.k), &root, &x_, &y_);
         const uint32_t smp = (uint32_t)*a.sample_dev + (uint32_t)path_sample(p, a.k);
         const tt_ray r = a.rays_in[i];
         const tt_hit h = a.hits[i];
@@ -667,7 +668,7 @@ __device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const in
     if (cont) {
         a.rays_out[slot] = nr;
         a.path_out[slot] = p;
-        a.root_out[slot] = root;
+        if (a.root_out) a.root_out[slot] = root;
     }
 }
 
@@ -1098,31 +1099,43 @@ __global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const
 
 // GUIDED: the guide's mixture, training records and roulette rule are compiled in
 // only for guided renders, so the plain kernel keeps its registers for occupancy.
+// Bound by HBM and, on the camera bounce, by VALU issue about equally (133M camera-bounce
+// paths: 77% of the issue slots, 3 TB/s), so a path's bytes are kept down: the throughput
+// travels with the ray by queue slot (read and written in order), the radiance is touched
+// only where a bounce adds some, the scene of a ray comes from its path id and is queued
+// for the traversal only when there are several, and the camera bounce's path ids are not
+// stored. Against state by path id, read and written on every bounce: 33.0 -> 29.1 ms of
+// shading in the 1080p, 64 spp, depth 16 render over 1.3M triangles (103.6 -> 99.6 ms,
+// traced), 76 VGPRs against 84. Gathering a block's hits before its misses, for fuller
+// waves, gave nothing (33.2 -> 33.8 ms).
 template <bool GUIDED>
 __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t i, const int32_t n) {
     bool cont = false, shadow = false;
     int32_t p = 0, root = 0;
     tt_ray nr{}, sr{};
+    float4 nthr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     f3 scontrib = F3(0, 0, 0);
     const SceneView &sv = a.sv;
     const float p_env = sv.env ? (sv.num_emit > 0 ? 0.5f : 1.0f) : 0.0f;
     const float p_emit = sv.num_emit > 0 ? 1.0f - p_env : 0.0f;
     if (i < n) {
-        p = a.path_in[i];
-        root = a.root_in[i];
-        int sid_;
+        // the camera bounce's state is the generated one: path p in slot p, throughput 1,
+        // roulette weight 1
+        const bool first = a.bounce == 0;
+        p = first ? i : a.path_in[i];
         int32_t x_, y_;
-        const int32_t local = pixel_of_slot(a.tab, path_slot(p, a.k), &sid_, &x_, &y_);
+        const int32_t local = pixel_of_slot(a.tab, path_slot(p, a.k), &root, &x_, &y_);
         const uint32_t smp = (uint32_t)*a.sample_dev + (uint32_t)path_sample(p, a.k);
         const tt_ray r = a.rays_in[i];
         const tt_hit h = a.hits[i];
-        // the camera bounce's state is the generated one: throughput 1, roulette weight 1
-        const bool first = a.bounce == 0;
-        const float4 tp = first ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : a.thr[p];
+        const float4 tp = first ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : a.thr_in[i];
         f3 thr = xyz(tp);
         const float last_pdf = tp.w;
         const bool last_delta = tp.w < 0.0f;
-        float4 Ls = first ? make_float4(1.0f, 0.0f, 0.0f, 0.0f) : a.L[p];   // x: roulette weight, yzw: radiance
+        // x: roulette weight, yzw: radiance. The weight belongs to guided renders: a plain
+        // bounce past the first touches the path's radiance only where it adds some.
+        float4 Ls = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+        if (GUIDED && !first) Ls = a.L[p];
         if (first) a.Lsh[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const f3 ro = F3(r.ox, r.oy, r.oz), rd = F3(r.dx, r.dy, r.dz);
         f3 add = F3(0, 0, 0);
@@ -1282,7 +1295,7 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
                             f3 no = point + (side > 0.0f ? ngf : ngf * -1.0f) * eps;
                             nr = {no.x, no.y, no.z, 0.0f, wi.x, wi.y, wi.z, 1e20f};
                             cont = true;
-                            a.thr[p] = make_float4(thr.x, thr.y, thr.z, delta ? -1.0f : pdf_b);
+                            nthr = make_float4(thr.x, thr.y, thr.z, delta ? -1.0f : pdf_b);
                             Ls.x = rr;
                             if (rec_b && !delta && pdf_b > 0.0f) {
                                 guide_inputs(a.gd, point, ns, wo, rec_b);
@@ -1302,25 +1315,29 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
                 }
             }
         }
-        if (maxc(add) > 0.0f) {
+        const bool adds = maxc(add) > 0.0f;
+        if (adds) {
             const int tc = GUIDED ? train_slot(a.gd, p) : -1;
             if (tc >= 0) credit(a.gd.rec, tc, a.bounce, a.max_depth, add, 16);
+            if (!GUIDED && !first) Ls = a.L[p];
             Ls.y += add.x;
             Ls.z += add.y;
             Ls.w += add.z;
         }
-        a.L[p] = Ls;   // the path's own slot: no atomics; k_resolve sums a pixel's paths
+        // the path's own slot: no atomics; k_resolve sums a pixel's paths
+        if (GUIDED || first || adds) a.L[p] = Ls;
     }
     int slot, sslot;
     block_append2(cont, &a.counts[a.nxt], shadow, &a.counts[a.scount], &slot, &sslot);
     if (cont) {
         a.rays_out[slot] = nr;
+        a.thr_out[slot] = nthr;
         a.path_out[slot] = p;
-        a.root_out[slot] = root;
+        if (a.root_out) a.root_out[slot] = root;
     }
     if (shadow) {
         a.srays[sslot] = sr;
-        a.sroot[sslot] = root;
+        if (a.sroot) a.sroot[sslot] = root;
         a.scontrib[sslot] = make_float4(scontrib.x, scontrib.y, scontrib.z, __int_as_float(p));
     }
 }
@@ -1741,15 +1758,17 @@ struct GuideRun {
     float first_loss = 0.0f;  // loss of the first Adam step
 };
 
-tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64) {
+tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64, bool roots) {
     RenderState *rs = s->rs;
-    if (rs && rs->cap >= cap && rs->pix_cap >= npix && (!fp64 || rs->acc64_cap >= npix)) return TT_OK;
+    if (rs && rs->cap >= cap && rs->pix_cap >= npix && (!fp64 || rs->acc64_cap >= npix) && (!roots || rs->roots))
+        return TT_OK;
     free_render_state(s);
     rs = new (std::nothrow) RenderState();
     if (!rs) return fail(TT_ERR_NOMEM, "render state: host allocation failed");
     s->rs = rs;
     rs->cap = cap;
     rs->pix_cap = npix;
+    rs->roots = roots;
     tt_status st = TT_OK;
     auto al = [&](void **p, size_t bytes, const char *what) {
         if (st == TT_OK) st = dev_alloc(s->ctx, p, bytes, what);
@@ -1757,15 +1776,15 @@ tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64) {
     for (int k = 0; k < 2; ++k) {
         al((void **)&rs->rays[k], (size_t)cap * sizeof(tt_ray), "render rays");
         al((void **)&rs->path[k], (size_t)cap * 4, "render path ids");
-        al((void **)&rs->root[k], (size_t)cap * 4, "render ray roots");
+        if (roots) al((void **)&rs->root[k], (size_t)cap * 4, "render ray roots");
+        al((void **)&rs->thr[k], (size_t)cap * 16, "render throughput");
     }
     al((void **)&rs->hits, (size_t)cap * sizeof(tt_hit), "render hits");
-    al((void **)&rs->thr, (size_t)cap * 16, "render throughput");
     al((void **)&rs->L, (size_t)cap * 16, "render radiance");
     al((void **)&rs->Lsh, (size_t)cap * 16, "render next-event radiance");
     for (int k = 0; k < 2; ++k) {
         al((void **)&rs->srays[k], (size_t)cap * sizeof(tt_ray), "render shadow rays");
-        al((void **)&rs->sroot[k], (size_t)cap * 4, "render shadow roots");
+        if (roots) al((void **)&rs->sroot[k], (size_t)cap * 4, "render shadow roots");
         al((void **)&rs->scontrib[k], (size_t)cap * 16, "render shadow contributions");
         al((void **)&rs->socc[k], (size_t)cap * 4, "render shadow flags");
     }
@@ -1862,11 +1881,12 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     sa.rays_out = rs->rays[nxt];
     sa.path_in = rs->path[cur];
     sa.path_out = rs->path[nxt];
-    sa.root_in = rs->root[cur];
     sa.root_out = rs->root[nxt];
     sa.sroot = rs->sroot[set];
     sa.hits = rs->hits;
-    sa.thr = rs->thr;
+    sa.thr = rs->thr[0];
+    sa.thr_in = rs->thr[cur];
+    sa.thr_out = rs->thr[nxt];
     sa.L = rs->L;
     sa.Lsh = rs->Lsh;
     sa.counts = rs->counts;
@@ -1942,7 +1962,7 @@ hipError_t launch_pass(tt_scene *s, RenderState *rs, const tt_render_params *p, 
     g.rays = rs->rays[0];
     g.path = rs->path[0];
     g.root = rs->root[0];
-    g.thr = rs->thr;
+    g.thr = rs->thr[0];
     g.L = rs->L;
     g.counts = rs->counts;
     hipLaunchKernelGGL(k_generate, dim3((unsigned)((cap + 255) / 256)), dim3(256), 0, hs, g);
@@ -2125,7 +2145,7 @@ tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const tt_
     // its own slot and the pass ends by adding a pixel's samples in sample order, in
     // both modes). Each bounce's launches last as long as their slowest waves, so the
     // fewer the passes the less that tail costs: by default up to 2^27 paths (256 B of
-    // state each, 34.4 GB) are in flight, guided renders with a frozen network included
+    // state each, 272 B with several scenes: 34.4 GB) are in flight, guided renders with a frozen network included
     // (about 232 B more per path for the network's inputs, mixture and slot list). Renders that train the network
     // default to about 8M paths: it learns between passes.
     int32_t k = 1;
@@ -2143,7 +2163,7 @@ tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const tt_
         while (k_after > 1 && (int64_t)k_after * npix > (1LL << 27)) --k_after;
         k_after = std::max(k_after, k);
     }
-    st = ensure_state(s, npix * k_after, npix, fp64);
+    st = ensure_state(s, npix * k_after, npix, fp64, nsc > 1);
     if (st != TT_OK) return st;
     RenderState *rs = s->rs;
     hipStream_t hs = ctx->stream;
@@ -2270,8 +2290,8 @@ tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const tt_
 void free_render_state(tt_scene *s) {
     RenderState *rs = s->rs;
     if (!rs) return;
-    void *ptrs[] = {rs->rays[0], rs->rays[1], rs->path[0], rs->path[1], rs->root[0], rs->root[1], rs->hits, rs->thr,
-                    rs->L, rs->Lsh, rs->srays[0], rs->srays[1], rs->sroot[0], rs->sroot[1], rs->scontrib[0],
+    void *ptrs[] = {rs->rays[0], rs->rays[1], rs->path[0], rs->path[1], rs->root[0], rs->root[1], rs->hits, rs->thr[0],
+                    rs->thr[1], rs->L, rs->Lsh, rs->srays[0], rs->srays[1], rs->sroot[0], rs->sroot[1], rs->scontrib[0],
                     rs->scontrib[1], rs->socc[0], rs->socc[1], rs->counts, rs->stats,
                     rs->sample_dev, rs->table, rs->acc, rs->acc64};
     for (void *q : ptrs)
