@@ -390,7 +390,7 @@ typedef struct tt_render_params {
     int32_t block;            /* traversal block size (0 = 64) */
     int32_t variant;          /* path-mode traversal loop: -1 speculative (default), 0 exact, 1 speculative */
     int32_t refill_camera;    /* traversal refill (see tt_trace_cfg) for the camera rays (0 = one wave per group) */
-    int32_t refill;           /* ... for every later extension and shadow launch (0 = persistent, 16) */
+    int32_t refill;           /* ... for every later extension and shadow launch (0 = persistent, 40) */
     int32_t tile;             /* path slots walk tile x tile pixel blocks (0 = 8; 1 = pixel rows; 2..32);
                                  the image does not depend on it */
 } tt_render_params;

@@ -71,7 +71,7 @@ RENDER_SPACE = {
     "use_graph": (False, True),
     "lds_stack": (16, 8, 24),           # traversal LDS stack entries per lane
     "block": (64, 128, 256),            # traversal block size
-    "refill": (16, 8, 32),              # persistent-wave refill of the later bounces
+    "refill": (40, 16, 24),             # persistent-wave refill of the later bounces
     "tile": (8, 4, 16),                 # path slots walk tile x tile pixel blocks
 }
 
