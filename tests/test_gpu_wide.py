@@ -42,8 +42,9 @@ def _mesh(tt, kind):
         v, t = _grid(20, 1.0, rng)
         v2, t2 = _grid(20, 4.0, rng)
         return tt.Mesh.from_arrays(*_join([(v, np.concatenate([t] * 4)), (v2, t2)]))
-    if kind == "piles":          # 60 coincident triangles at each of 200 places: large leaves
-        v = rng.normal(0, 4, (200, 1, 3)) + rng.normal(0, 2, (200, 3, 3))
+    if kind in ("piles", "spread"):   # 60 coincident triangles at each place: large leaves
+        n = 200 if kind == "piles" else 12000   # (a tree past the packed records' size)
+        v = rng.normal(0, 4, (n, 1, 3)) + rng.normal(0, 2 if n == 200 else 0.2, (n, 3, 3))
         v = np.repeat(v, 60, axis=0).reshape(-1, 3)
         return tt.Mesh.from_arrays(v.astype(np.float32), np.arange(len(v), dtype=np.int32).reshape(-1, 3))
     if kind == "line":           # triangles along a line: a deep tree, many pending children
@@ -106,7 +107,7 @@ def _rays(mesh, seed):
     return np.concatenate(out)
 
 
-@pytest.mark.parametrize("kind", ["layers", "hills", "coincident", "piles", "line"])
+@pytest.mark.parametrize("kind", ["layers", "hills", "coincident", "piles", "line", "spread"])
 def test_four_child_walk_matches_oracle(tt, oracle, ctx, kind):
     print(f"four-child walk: {kind}", file=sys.stderr, flush=True)
     mesh = _mesh(tt, kind)

@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                 st.clear();
                 redo = !fits;
                 leaf = leaf2 = 0;
-                node = fits ? 3 * (a.ray_root ? a.ray_root[rid] : 0) : kSentinel;
+                node = fits ? a.wide_step * (a.ray_root ? a.ray_root[rid] : 0) : kSentinel;
                 hit_t = next_t = tmax;
                 hit_rec = -1;
                 cull = fb(tmax * 1.0009765625f);
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                 const float4 A = tp[0], B = tp[1], C = tp[2];
                 float t, u, v;
                 const bool end = fb(C.w) < 0;
-                leaf = end ? leaf2 : leaf + 3;
+                leaf = end ? leaf2 : leaf + a.wide_step;
                 leaf2 = end ? 0 : leaf2;
                 if (tri_test<TRI>(A, B, C, ox, oy, oz, dx, dy, dz, tmin, ANY ? hit_t : bf(cull), &t, &u, &v)) {
                     if (ANY) {

@@ -1,7 +1,8 @@
 // The four-child tree k_trace_wide walks, built on the GPU from the two-child SBVH when a
 // scene is created.
 //
-// One array of 48-byte records (three 16-byte units), nodes and triangles alike; a
+// One array of records, nodes and triangles alike: 48 bytes (three 16-byte units) of
+// content, 48 or 64 bytes apart (by the tree's size: build_wide); a
 // reference is a unit index below 2^30, with the sign bit set for a leaf. The scenes'
 // roots come first; a node's children lie together, inner nodes first, then the leaves'
 // triangle records. The walk is bound by VALU issue and by vector memory lane loads, so a
@@ -34,7 +35,7 @@
 namespace tt {
 namespace {
 
-constexpr int kMaxOffset = 42;   // largest record offset of a slot (126 units)
+constexpr int kMaxOffset = 127;   // largest unit offset of a slot
 constexpr int32_t kRingEnd = 0x7FFFFFFF;   // no unit index
 
 struct WideBuild {
@@ -42,7 +43,8 @@ struct WideBuild {
     const float4 *tris;
     const int32_t *roots;   // two-child roots of the scenes
     int32_t nroots;
-    uint4 *wide;            // [3 * record]
+    uint4 *wide;            // [step * record]
+    int32_t step;           // units from one record to the next
     // breadth-first list of the nodes: record, and place in the two-child tree (node * 2 +
     // child; roots: unused)
     int2 *list;
@@ -105,13 +107,13 @@ __device__ bool add_children(const WideBuild &b, int32_t node, const Child *in, 
 
 // Whether the leaves among c[0, n) can be addressed: the inner children and all leaves but
 // the largest lie before it.
-__device__ bool leaves_fit(const Child *c, int n) {
+__device__ bool leaves_fit(const Child *c, int n, int32_t step) {
     int64_t before = 0, most = 0;
     for (int k = 0; k < n; ++k) {
         before += c[k].count ? c[k].count : 1;
         most = max(most, (int64_t)c[k].count);
     }
-    return before - most <= kMaxOffset;
+    return (before - most) * step <= kMaxOffset;
 }
 
 __device__ int wave_scan(int v, int *total) {   // exclusive sum over the wave's lanes
@@ -126,18 +128,19 @@ __device__ int wave_scan(int v, int *total) {   // exclusive sum over the wave's
 
 __device__ void copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_t place, int32_t at, bool last) {
     const float4 *t = b.tris + (int64_t)~ref * 3;
-    float4 *to = reinterpret_cast<float4 *>(b.wide) + (int64_t)at * 3;
     for (int i = 0; i < count; ++i) {
+        const int32_t unit = b.step * (at + i);
+        float4 *to = reinterpret_cast<float4 *>(b.wide) + unit;
         float4 e1 = t[3 * i + 1], e2 = t[3 * i + 2];
         const int32_t id = __float_as_int(t[3 * i].w);
         // the record before this one in the ring; the first closes it (k_wide_rings)
-        int32_t link = id >= 0 && id < b.ids ? atomicExch(&b.last_of[id], 3 * (at + i)) : 3 * (at + i);
+        int32_t link = id >= 0 && id < b.ids ? atomicExch(&b.last_of[id], unit) : unit;
         if (link < 0) link = kRingEnd;
         e1.w = __int_as_float(place);
         e2.w = __int_as_float(link | (last && i + 1 == count ? (int32_t)0x80000000 : 0));
-        to[3 * i] = t[3 * i];
-        to[3 * i + 1] = e1;
-        to[3 * i + 2] = e2;
+        to[0] = t[3 * i];
+        to[1] = e1;
+        to[2] = e2;
     }
 }
 
@@ -185,7 +188,7 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
             const int4 ch = reinterpret_cast<const int4 *>(b.nodes)[(int64_t)(p >> 1) * 4 + 3];
             bad = !add_children(b, (p & 1) ? ch.y : ch.x, &self, c, n);
         }
-        if (!bad && n == 2 && !leaves_fit(c, n)) {
+        if (!bad && n == 2 && !leaves_fit(c, n, b.step)) {
             // two large leaves: one slot for both
             c[0].ref2 = c[1].ref;
             c[0].count2 = c[1].count;
@@ -213,7 +216,7 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
                 if (k != best) trial[t++] = c[k];
             for (int k = 0; k < m; ++k) trial[t++] = two[k];
             if (bad) break;
-            if (!leaves_fit(trial, t)) {
+            if (!leaves_fit(trial, t, b.step)) {
                 shut[best] = true;
                 continue;
             }
@@ -294,26 +297,27 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
     for (int k = 0; k < n; ++k) {
         if (c[k].count == 0) {
             b.list[node0 + k] = make_int2(rec0 + k, c[k].place);
-            offsets |= (uint32_t)(3 * off) << (8 * k);
+            offsets |= (uint32_t)(b.step * off) << (8 * k);
             ++off;
             continue;
         }
-        offsets |= (uint32_t)(128 | 3 * off) << (8 * k);
+        offsets |= (uint32_t)(128 | b.step * off) << (8 * k);
         copy_leaf(b, c[k].ref, c[k].count, c[k].place, rec0 + off, c[k].count2 == 0);
         if (c[k].count2) copy_leaf(b, c[k].ref2, c[k].count2, c[k].place2, rec0 + off + c[k].count, true);
         off += c[k].count + c[k].count2;
     }
     if (no_leaf) {
         // no edges (never accepted), no triangle, its own ring, the end of its leaf
-        float4 *to = reinterpret_cast<float4 *>(b.wide) + ((int64_t)rec0 + off) * 3;
+        const int32_t unit = b.step * (rec0 + off);
+        float4 *to = reinterpret_cast<float4 *>(b.wide) + unit;
         to[0] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
         to[1] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
-        to[2] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(3 * (rec0 + off) | (int32_t)0x80000000));
+        to[2] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(unit | (int32_t)0x80000000));
     }
-    for (int k = n; k < 4; ++k) offsets |= (uint32_t)(128 | 3 * inner) << (8 * k);
-    uint4 *w = b.wide + (int64_t)self_rec * 3;
+    for (int k = n; k < 4; ++k) offsets |= (uint32_t)(128 | b.step * inner) << (8 * k);
+    uint4 *w = b.wide + b.step * self_rec;
     w[0] = make_uint4(__float_as_uint(lo[0]), __float_as_uint(lo[1]), __float_as_uint(lo[2]),
-                      3u * (uint32_t)rec0);
+                      (uint32_t)(b.step * rec0));
     w[1] = make_uint4(offsets, code[0] | code[1] << 8 | code[2] << 16, planes[0][0], planes[0][1]);
     w[2] = make_uint4(planes[1][0], planes[1][1], planes[2][0], planes[2][1]);
 }
@@ -367,6 +371,14 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     // nodes at most as many as the two-child tree has; units below 2^30
     const int64_t recs = s->num_nodes + s->num_tris;
     if (s->num_nodes == 0 || recs >= (1 << 30) / 3) return TT_OK;
+    // A tree past the L2s (8 of 4 MB) takes 64 bytes per record: a record then lies in one
+    // 64-byte piece of memory instead of 1.5, which is what a miss fetches; a smaller one
+    // stays packed. Measured with 48 / 64 bytes: any hit on soup, 1M rays, 223k records 378 /
+    // 373 us, 448k 460 / 455, 909k 525 / 490, 1.6M 580 / 544; 1080p, 64 spp path tracing over
+    // 1.76M records 96.2 / 91.9 ms; 540p guided render over 110k records 12.67 / 12.92 ms; 360p,
+    // 4 spp over 110k records 2.60 / 2.69 ms, over 439k 3.60 / 3.68.
+    constexpr int64_t kPacked = (32 << 20) / 48;
+    const int32_t step = recs > kPacked && recs < (1 << 30) / 4 ? 4 : 3;
     constexpr double kShort = 20.0;
     if (std::none_of(roots.begin(), roots.end(), [&](int32_t r) { return costs_more_than(dev_nodes, r, kShort); }))
         return TT_OK;
@@ -385,7 +397,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     }
     if (!(bound < 0x1p60)) return TT_OK;
     void *mem = nullptr, *tmp = nullptr;
-    const size_t bytes = (size_t)recs * 48;
+    const size_t bytes = (size_t)recs * step * 16;
     // triangle ids (0 .. max(id)): those of the scene's mesh, or of as many records as there are
     const int32_t ids = (int32_t)std::max<int64_t>(s->num_orig_tris, s->num_tris);
     const size_t list_bytes = (size_t)s->num_nodes * 8, root_bytes = roots.size() * 4;
@@ -403,6 +415,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     b.list = reinterpret_cast<int2 *>(b.state + 4);
     int32_t *d_roots = b.state + 4 + 2 * s->num_nodes;
     b.roots = d_roots;
+    b.step = step;
     b.nroots = (int32_t)roots.size();
     b.last_of = d_roots + roots.size();
     b.ids = ids;
@@ -436,6 +449,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
         return err == hipSuccess ? TT_OK : fail(TT_ERR_DEVICE, std::string("scene tree: ") + hipGetErrorString(err));
     }
     s->wide = mem;
+    s->wide_step = step;
     s->wide_bound = (float)(bound * (1.0 + 4.0 / 255.0)) * 1.0001f;
     s->bytes += bytes;
     return TT_OK;
