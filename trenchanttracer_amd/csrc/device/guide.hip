@@ -153,6 +153,7 @@ struct InferArgs {
     const __bf16 *w[4];
     const float *bias[4];
     float *raw;
+    int32_t raw_ld;   // columns written, and row stride of raw: kGuideNOutPad16, or the kGuideNOut real ones
     int64_t n;
     const int32_t *n_dev;
     // if set: row r reads its inputs from and writes its outputs to row slot_of[r] of in
@@ -331,9 +332,10 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(InferArgs a) {
         if (dst >= 0) {
 #pragma unroll
             for (int t = 0; t < kGuideNOutPad16 / 16; ++t)
-                *reinterpret_cast<float4 *>(a.raw + dst * kGuideNOutPad16 + 16 * t + 4 * lq) =
-                    make_float4(out[t][0] + b4[16 * t + 4 * lq], out[t][1] + b4[16 * t + 4 * lq + 1],
-                                out[t][2] + b4[16 * t + 4 * lq + 2], out[t][3] + b4[16 * t + 4 * lq + 3]);
+                if (16 * t + 4 * lq < a.raw_ld)
+                    *reinterpret_cast<float4 *>(a.raw + dst * a.raw_ld + 16 * t + 4 * lq) =
+                        make_float4(out[t][0] + b4[16 * t + 4 * lq], out[t][1] + b4[16 * t + 4 * lq + 1],
+                                    out[t][2] + b4[16 * t + 4 * lq + 2], out[t][3] + b4[16 * t + 4 * lq + 3]);
         }
         slot = slot_next;
     }
@@ -1118,9 +1120,10 @@ hipError_t guide_forward(tt_guide *g, int64_t n, const int32_t *n_dev, hipStream
 // Inference over the first n rows of g->batch.in (device count n_dev optional):
 // the fused kernel, raw outputs (fp32, 48 wide) into g->batch.raw.
 hipError_t guide_infer(tt_guide *g, const float *in, float *raw, int64_t n, const int32_t *n_dev, hipStream_t s,
-                       const int32_t *slot_of, bool store_acts) {
+                       const int32_t *slot_of, bool store_acts, int32_t raw_ld) {
     InferArgs a{};
     a.in = in;
+    a.raw_ld = raw_ld;
     a.slot_of = slot_of;
     if (store_acts)   // the training forward pass: hidden activations into the batch (the
                       // first layer's weight gradient recomputes the features)
@@ -1411,8 +1414,11 @@ tt_status tt_guide_forward(tt_guide *g, const float *inputs, int64_t n, float *r
     if (st != TT_OK) return st;
     hipStream_t s = g->ctx->stream;
     TT_HIPG(hipMemcpyAsync(g->batch.in, inputs, (size_t)n * kGuideIn * 4, hipMemcpyHostToDevice, s), "copy inputs");
-    TT_HIPG(guide_infer(g, g->batch.in, g->batch.raw, n, nullptr, s), "guide inference");
-    return copy_raw_out(g, n, raw_out, s);
+    // packed rows on the device: they go to the caller's buffer as they are
+    TT_HIPG(guide_infer(g, g->batch.in, g->batch.raw, n, nullptr, s, nullptr, false, kGuideNOut), "guide inference");
+    TT_HIPG(hipMemcpyAsync(raw_out, g->batch.raw, (size_t)n * kGuideNOut * 4, hipMemcpyDeviceToHost, s), "copy out");
+    TT_HIPG(hipStreamSynchronize(s), "sync");
+    return TT_OK;
 }
 
 tt_status tt_debug_guide_forward_unfused(tt_guide *g, const float *inputs, int64_t n, float *raw_out) {

@@ -145,9 +145,11 @@ hipError_t guide_forward(tt_guide *g, int64_t n, const int32_t *n_dev, hipStream
 // slot_of (may be null): row r of the inference reads inputs and writes outputs at
 // row slot_of[r] of in and raw (a compacted list of the rows needed); rows up to
 // min(*n_dev, n). store_acts: also write the features and hidden activations into
-// g->batch (training)
+// g->batch (training). raw_ld: columns written and row stride of raw, kGuideNOutPad16 or,
+// without the padding, kGuideNOut
 hipError_t guide_infer(tt_guide *g, const float *in, float *raw, int64_t n, const int32_t *n_dev, hipStream_t s,
-                       const int32_t *slot_of = nullptr, bool store_acts = false);
+                       const int32_t *slot_of = nullptr, bool store_acts = false,
+                       int32_t raw_ld = kGuideNOutPad16);
 hipError_t guide_train_rows(tt_guide *g, int64_t n, hipStream_t s);
 tt_status guide_alloc_batch(tt_guide *g, int64_t rows);
 tt_status guide_alloc_infer(tt_guide *g, int64_t rows);
