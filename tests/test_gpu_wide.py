@@ -150,6 +150,36 @@ def test_four_child_walk_of_several_trees(tt, ctx):
     batch.close()
 
 
+@pytest.mark.parametrize("tris", [30, 20000])   # two-child loop, four-child walk
+def test_few_rays_in_small_groups(tt, ctx, tris):
+    """Counts around the steps of the group size (1 to 64 rays): the records of a launch of
+    full groups, and nothing written past the end."""
+    mesh = tt.Mesh.soup(tris, seed=4, mu=float(np.log(0.3))) if tris == 30 else tt.Mesh.soup(tris, seed=6)
+    scene = tt.DeviceScene(ctx, mesh, tt.BVH.build(mesh))
+    total = 200_003
+    d = tt.DeviceBuffer.from_array(ctx, tt.rays_incoherent(mesh, total, seed=8))
+    h = tt.DeviceBuffer(ctx, (total + 64) * 16)
+    f = tt.DeviceBuffer(ctx, (total + 64) * 4)
+
+    def trace(n, cfg):
+        h.upload(np.full((n + 64, 4), 7.0, np.float32))
+        f.upload(np.full(n + 64, 7, np.int32))
+        scene.trace_closest(d, n, h, cfg)
+        scene.trace_any(d, n, f, cfg)
+        ctx.sync()
+        return h.download((n + 64, 4), np.int32), f.download(n + 64, np.int32)
+    want, hit = trace(total, None)
+    for n in (1, 2, 63, 64, 65, 2047, 2048, 2049, 4096, 4097, 65_535, 65_537, 131_072, 131_073):
+        print(f"small groups: {n} rays", file=sys.stderr, flush=True)
+        for cfg in (None, tt.trace_cfg(1, 8, 256), tt.trace_cfg(0, 16, 64, refill=24), tt.trace_cfg(1, 16, 64, reorder=1)):
+            got, flags = trace(n, cfg)
+            assert np.array_equal(got[:n], want[:n]) and np.array_equal(flags[:n], hit[:n])
+            assert (got[n:].view(np.float32) == 7.0).all() and (flags[n:] == 7).all()
+    for b in (d, h, f):
+        b.free()
+    scene.close()
+
+
 def test_sweeps_trace_every_ray_once(tt, ctx):
     """refill 0 traces the range in parts; ray counts below, at and past one group per
     resident wave and one part, ragged: the records of the persistent launch, and nothing

@@ -32,6 +32,7 @@ struct TraceArgs {
     int32_t refill;        // a wave takes new rays once this many of its lanes are idle (1..64)
     int32_t sweep;         // if set: the range is traced in parts of this many groups per wave ...
     int32_t sweep_waves;   // ... and this many waves
+    int32_t spread;        // if set: groups shrink to 2^k < 64 rays while there are at most 2^spread of them
     const uint32_t *order; // if set: the r-th ray traced is ray order[r] (a permutation of 0..n-1)
     // node-fetch probe (closest-hit loop): per ray the counts of node visits,
     // triangle tests and leaf visits, and from rec_off[ray] (32-bit words) the 4-bit

@@ -283,6 +283,13 @@ __device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, 
     return false;
 }
 
+// log2 of the rays of a group (TraceArgs::spread), uniform.
+__device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
+    if (!spread || n == 0u) return 6;
+    const uint32_t full = (n - 1u) >> spread;
+    return full ? min(6, 32 - __clz((int)full)) : 0;
+}
+
 // Four-child walk. What bounds it: VALU issue first, vector memory lane loads second. On
 // the 1M-triangle soup (8.3M rays in Morton order) the two-child while-while loop kept VALU
 // issue 90% and the address path 82% busy, with 32% of the lanes active: 1.85e9 VALU
@@ -324,7 +331,8 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
     // ray. Each ray's traversal is the same as with one ray per lane. The wave's number is
     // read from its first lane, so that everything uniform stays in scalar registers and
     // the loops below branch on scalars.
-    const uint32_t groups = (n + 63u) >> 6;
+    const int gs = group_bits(n, a.spread);
+    const uint32_t groups = (uint32_t)(((uint64_t)n + (1u << gs) - 1u) >> gs);
     const uint32_t w = vb * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t waves = max(1u, min(gridDim.x * (blockDim.x >> 6), groups)), first = w, last = groups;
     if (a.sweep) {
@@ -335,7 +343,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
     }
     // whole waves only: nothing below synchronises the block
     if (first >= last || (!a.sweep && w >= waves)) return;
-    const uint32_t total = ((last - first + waves - 1u) / waves) * 64u;   // the wave's sequence positions
+    const uint32_t total = ((last - first + waves - 1u) / waves) << gs;   // the wave's sequence positions
     const unsigned long long below = (1ull << lane) - 1ull;
 
     // one private array serves both walks
@@ -391,7 +399,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
         if (take && done) {
             const uint32_t q = cursor + (uint32_t)__popcll(m & below);
             if (q < total) {
-                const uint32_t r = ((q >> 6) * waves + first) * 64u + (q & 63u);
+                const uint32_t r = (((q >> gs) * waves + first) << gs) + (q & ((1u << gs) - 1u));
                 if (r < n) rid = (int)(a.order ? a.order[r] : r);
             }
             if (rid >= 0) {
@@ -591,12 +599,13 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
         if (a.reset1) *a.reset1 = 0;
     }
     // the launch form of k_trace_wide
-    const int64_t groups = (n + 63) >> 6;
+    const int gs = group_bits((uint32_t)max((int64_t)0, n), a.spread);
+    const int64_t groups = (n + (1 << gs) - 1) >> gs;
     const int64_t waves_all = (int64_t)gridDim.x * (blockDim.x >> 6);
     const int64_t waves = max((int64_t)1, min(waves_all, groups));
     const int64_t w = (int64_t)vb * (blockDim.x >> 6) + (tid >> 6);
     if (w >= waves) return;   // whole waves only: nothing below synchronises the block
-    const int64_t total = ((groups - w + waves - 1) / waves) * 64;   // the wave's sequence positions
+    const int64_t total = ((groups - w + waves - 1) / waves) << gs;   // the wave's sequence positions
     const unsigned long long below = (1ull << lane) - 1ull;
 
     int spill[kStackCap - S];
@@ -646,7 +655,7 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
         if (take && done) {
             const int64_t q = cursor + __popcll(m & below);
             if (q < total) {
-                const int64_t r = ((q >> 6) * waves + w) * 64 + (q & 63);
+                const int64_t r = (((q >> gs) * waves + w) << gs) + (q & ((1 << gs) - 1));
                 if (r < n) rid = a.order ? (int64_t)a.order[r] : r;
             }
             if (rid >= 0) {
@@ -813,13 +822,16 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
 // one group per wave is a launch of one wave per group.
 template <class K>
 hipError_t launch_k(K kernel, TraceArgs a, bool persistent, int block, size_t lds, int num_cus, hipStream_t s) {
-    int64_t grid = (a.n + block - 1) / block;
+    // lanes of a group, as the kernel sets them (group_bits)
+    int64_t rays = 64;
+    while (a.spread && rays > 1 && a.n <= (rays / 2) << a.spread) rays /= 2;
+    int64_t grid = ((a.n + rays - 1) / rays + block / 64 - 1) / (block / 64);
     if (persistent) {
         int per_cu = 0;
         hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds);
         if (e != hipSuccess) return e;
         const int64_t resident = (int64_t)std::max(1, per_cu) * std::max(1, num_cus);
-        const int64_t groups = (a.n + 63) / 64, waves = resident * (block / 64);
+        const int64_t groups = (a.n + rays - 1) / rays, waves = resident * (block / 64);
         if (a.sweep && groups > waves) {
             a.sweep_waves = (int32_t)waves;
             const int64_t part = waves * a.sweep;
@@ -912,6 +924,16 @@ hipError_t launch_trace(const TraceArgs &a, int variant, bool any, int lds_stack
     // refill 0: one wave per 64-ray group; 1..64: persistent waves with that threshold
     const bool persistent = refill > 0;
     b.refill = persistent ? (refill > 64 ? 64 : refill) : 64;
+    // Few rays are spread over the chip: with fewer than 64 for each of 8 waves per CU a group
+    // shrinks: a wave takes as many rounds as its rays ask for in turn, fewer rays ask for
+    // fewer, and there is room for more waves. Any-hit rays in 223k records,
+    // closest-hit rays in 550k, us, groups of 64 / 4 waves per CU / 8 / 16 / 32: 1000 rays 113
+    // / 75 / 73 / 76 / 73 and 143 / 97 / 96 / 102 / 98; 10000: 138 / 123 / 116 / 117 / 125 and
+    // 212 / 180 / 181 / 163 / 164; 50000: 190 / 188 / 181 / 175 / 182 and 273 / 272 / 281 / 266
+    // / 268; 200000 (64 rays at 8 waves): 245 / 248 / 247 / 247 / 261 and 321 / 322 / 320 / 321
+    // / 337. Guided render 12.75 / 12.58 / 12.58 / 12.69 / 13.29 ms, room of 20 triangles 2089
+    // / 2091 / 2096 / 2106 / 2143 us.
+    for (b.spread = 0; 8LL * std::max(1, num_cus) >> (b.spread + 1);) ++b.spread;
     // ray indices are 32-bit in the kernel: more rays go in several launches (a device-side
     // count or an order comes with fewer)
     constexpr int64_t kPart = (int64_t)1 << 30;
