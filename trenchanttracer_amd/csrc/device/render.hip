@@ -50,7 +50,9 @@ struct RenderState {
     tt_ray *srays[2] = {nullptr, nullptr};     // next-event rays
     float4 *scontrib[2] = {nullptr, nullptr};  // contribution (rgb) and path id (w, as int bits)
     int32_t *socc[2] = {nullptr, nullptr};     // any-hit flags
-    int32_t *counts = nullptr;   // [0], [1] queues, [2 + (b & 3)] next-event queue of bounce b
+    // counters of queues 0 and 1 and of next-event queue 2 + (b & 3) of bounce b (kQueue words
+    // each); then the number of camera rays
+    int32_t *counts = nullptr;
     unsigned long long *stats = nullptr;  // [0] extension rays, [1] shadow rays
     float *acc = nullptr;        // per pixel rgb
     double *acc64 = nullptr;     // per pixel rgb (FP64 accumulation)
@@ -211,6 +213,9 @@ __device__ __forceinline__ int32_t path_slot(int32_t p, int32_t k) { return p / 
 __device__ __forceinline__ int32_t path_sample(int32_t p, int32_t k) { return p % k; }
 __device__ __forceinline__ int64_t path_id(int32_t q, int32_t s, int32_t k) { return (int64_t)q * k + s; }
 
+constexpr int kQueue = kSegs * kSegStride;   // counter words of a queue
+constexpr int kCameraCount = 6 * kQueue;     // the word after those of the six queues
+
 struct GenArgs {
     const SceneTable *tab;
     int32_t npix, mode, k;   // k samples per pixel in flight: path id = slot * k + j (pixel_of_slot)
@@ -227,9 +232,7 @@ __global__ __launch_bounds__(256) void k_generate(GenArgs a) {
     const int32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     const int32_t npix = a.npix;
     if (p == 0) {
-        a.counts[0] = npix * a.k;
-        a.counts[1] = 0;
-        a.counts[2] = 0;
+        a.counts[kCameraCount] = npix * a.k;
     }
     if (p >= npix * a.k) return;
     int sid;
@@ -339,7 +342,7 @@ struct GeomArgs {
     const tt_ray *rays;
     tt_hit *hits;        // closest: replaced when a primitive is strictly nearer
     int32_t *occ;        // any: set when a primitive lies inside the ray interval
-    const int32_t *n_dev;
+    Queue queue;
     const tt_geometry *geoms;
     int32_t num_geoms;
 };
@@ -348,8 +351,10 @@ struct GeomArgs {
 // (src/core/RenderKernel.cu:38-61); the nearest primitive below tmax wins when
 // strictly nearer than the triangle hit (a miss carries t = tmax).
 __global__ __launch_bounds__(256) void k_geom_hits(GeomArgs a) {
-    const int32_t n = *a.n_dev;
-    for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int32_t n = queue_span(a.queue);
+    for (int32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int32_t i = queue_slot(a.queue, k);
+        if (i < 0) continue;
         const tt_ray r = a.rays[i];
         const tt_hit h = a.hits[i];
         const f3 o = F3(r.ox, r.oy, r.oz), d = F3(r.dx, r.dy, r.dz);
@@ -367,9 +372,10 @@ __global__ __launch_bounds__(256) void k_geom_hits(GeomArgs a) {
 }
 
 __global__ __launch_bounds__(256) void k_geom_occluded(GeomArgs a) {
-    const int32_t n = *a.n_dev;
-    for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (a.occ[i]) continue;
+    const int32_t n = queue_span(a.queue);
+    for (int32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int32_t i = queue_slot(a.queue, k);
+        if (i < 0 || a.occ[i]) continue;
         const tt_ray r = a.rays[i];
         const f3 o = F3(r.ox, r.oy, r.oz), d = F3(r.dx, r.dy, r.dz);
         for (int32_t k = 0; k < a.num_geoms; ++k)
@@ -478,9 +484,9 @@ struct ShadeArgs {
     float4 *thr_out;
     float4 *L;
     float4 *Lsh;       // zeroed for every path on the camera bounce
-    int32_t *counts;
-    int32_t cur, nxt;
-    int32_t scount;    // counts[scount]: this bounce's next-event queue
+    Queue queue;                       // of rays_in
+    int32_t *out_counts, *sh_counts;   // of rays_out and srays
+    int32_t seg;                       // capacity of their segments
     tt_ray *srays;
     float4 *scontrib;
     float *acc;
@@ -492,6 +498,24 @@ struct ShadeArgs {
     uint32_t seed;
     float inv_spp, pi, two_pi;
 };
+
+// The slots of a shade block, *n from *first on (at most kAppendBlock; false: none): a block
+// of the camera rays, or block b / kSegs of segment b % kSegs.
+__device__ __forceinline__ bool shade_block(const ShadeArgs &a, int32_t *first, int32_t *n) {
+    int32_t at = (int32_t)blockIdx.x, s = 0;
+    if (a.queue.seg) {
+        s = at % kSegs;
+        at /= kSegs;
+    }
+    at *= kAppendBlock;
+    *first = s * a.queue.seg + at;
+    // read before any atomic, so as a scalar: from the scalar cache, not from the lines the
+    // blocks' adds pass between the XCDs (1080p shading: 33 ms instead of 7)
+    const int32_t end = a.queue.counts[s * kSegStride];
+    *n = end - at;
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.stats[0], (unsigned long long)queue_total(a.queue));
+    return *n > 0;
+}
 
 // hdrSample (HDRKernel.cuh:6-42): nearest texel, x2; the row index is clamped
 // (the reference reads one row past the end for d.y near -1 with its PI).
@@ -517,13 +541,13 @@ __device__ f3 env_reference(const SceneView &sv, f3 d, float pi, float two_pi) {
 }
 
 // ------------------------------------------------------------------ reference shade
-// One slot of the hit queue (i >= n: no path; the thread still joins the block's
+// One slot of the hit queue (i < 0: no path; the thread still joins the block's
 // queue append).
-__device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const int32_t i, const int32_t n) {
+__device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const int32_t i) {
     bool cont = false;
     int32_t p = 0, root = 0;
     tt_ray nr{};
-    if (i < n) {
+    if (i >= 0) {
         p = a.path_in[i];
         int32_t x_, y_;
         const int32_t local = pixel_of_slot(a.tab, path_slot(p, a.k), &root, &x_, &y_);
@@ -664,8 +688,10 @@ __device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const in
         if (finish) a.L[p] = make_float4(Lp.x, Lp.y, Lp.z, 0.0f);
     }
     int slot, unused;
-    block_append2(cont, &a.counts[a.nxt], false, nullptr, &slot, &unused);
+    const int s = (int)(blockIdx.x % kSegs);
+    block_append2(cont, &a.out_counts[s * kSegStride], false, nullptr, &slot, &unused);
     if (cont) {
+        slot += s * a.seg;
         a.rays_out[slot] = nr;
         a.path_out[slot] = p;
         if (a.root_out) a.root_out[slot] = root;
@@ -677,10 +703,9 @@ __device__ __forceinline__ void shade_reference_one(const ShadeArgs &a, const in
 // queue would save those blocks' launch but takes the shade kernels from 73 to 97
 // VGPRs (6 to 4 waves per SIMD), which costs more at the full early bounces.
 __global__ __launch_bounds__(kAppendBlock) void k_shade_reference(ShadeArgs a) {
-    const int32_t n = a.counts[a.cur];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.stats[0], (unsigned long long)n);
-    if ((int64_t)blockIdx.x * kAppendBlock >= n) return;
-    shade_reference_one(a, (int32_t)(blockIdx.x * kAppendBlock + threadIdx.x), n);
+    int32_t first, n;
+    if (!shade_block(a, &first, &n)) return;
+    shade_reference_one(a, (int32_t)threadIdx.x < n ? first + (int32_t)threadIdx.x : -1);
 }
 
 // ------------------------------------------------------------------ path mode
@@ -968,11 +993,10 @@ struct GuideInArgs {
     SceneView sv;
     const tt_ray *rays;
     const tt_hit *hits;
-    const int32_t *counts;
-    int32_t cur;
-    float *in;          // [slot][9], written for the guided slots
-    uint64_t *mask;     // [slot / 64]: bit slot % 64 set where the vertex is guided
-    int32_t *block_n;   // [block]: guided slots of each block's span
+    Queue queue;
+    float *in;          // [row][9], written for the guided rows (row: position in the queue's sequence)
+    uint64_t *mask;     // [row / 64]: bit row % 64 set where the vertex is guided
+    int32_t *block_n;   // [block]: guided rows of each block's span
     const int32_t *given;   // check hook only: the guided flag of each slot (inputs already in in)
 };
 
@@ -982,11 +1006,13 @@ __device__ __forceinline__ bool guide_eligible(const tt_material &m, float min_r
     return m.type == TT_MAT_DIFFUSE || (m.type == TT_MAT_CONDUCTOR && m.roughness >= min_rough);
 }
 
-// Whether slot i's vertex is guided; if so, its network inputs into a.in[i].
+// Whether row i's vertex is guided; if so, its network inputs into a.in[i].
 __device__ __forceinline__ bool guide_vertex_inputs(const GuideInArgs &a, int64_t i) {
-    const tt_hit h = a.hits[i];
+    const int32_t slot = queue_slot(a.queue, (int32_t)i);
+    if (slot < 0) return false;
+    const tt_hit h = a.hits[slot];
     if (h.tri_id == -1) return false;
-    const tt_ray r = a.rays[i];
+    const tt_ray r = a.rays[slot];
     const f3 rd = F3(r.dx, r.dy, r.dz), wo = rd * -1.0f;
     const f3 point = F3(r.ox, r.oy, r.oz) + rd * h.t;
     const Surf sf = surface_path(a.sv, h, point);
@@ -1017,7 +1043,7 @@ __device__ __forceinline__ int64_t guide_span(int32_t n) {
 template <bool GIVEN>
 __global__ __launch_bounds__(256) void k_guide_inputs(GuideInArgs a) {
     __shared__ int32_t wc[4];
-    const int32_t n = a.counts[a.cur];
+    const int32_t n = queue_span(a.queue);
     const int64_t span = guide_span(n);
     const int64_t lo = (int64_t)blockIdx.x * span, hi = min((int64_t)n, lo + span);
     const int wave = threadIdx.x >> 6, lane = __lane_id();
@@ -1067,11 +1093,11 @@ __device__ __forceinline__ void scan_counts(int32_t *off, int64_t nb, int32_t *t
 // block adds the guided counts of the blocks before it (at most 16 per CU, in a fixed
 // order) for its first row, then walks its span 256 slots at a time; the last block
 // writes the row total.
-__global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const int32_t *block_n,
-                                                     const int32_t *n_dev, int32_t *slot_of, int32_t *total) {
+__global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const int32_t *block_n, Queue queue,
+                                                     int32_t *slot_of, int32_t *total) {
     __shared__ int32_t part[4];
     __shared__ int32_t wc[2][4];
-    const int32_t n = *n_dev;
+    const int32_t n = queue_span(queue);
     const int64_t span = guide_span(n);
     const int64_t lo = (int64_t)blockIdx.x * span, hi = min((int64_t)n, lo + span);
     const int wave = threadIdx.x >> 6, lane = __lane_id();
@@ -1109,7 +1135,7 @@ __global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const
 // traced), 76 VGPRs against 84. Gathering a block's hits before its misses, for fuller
 // waves, gave nothing (33.2 -> 33.8 ms).
 template <bool GUIDED>
-__device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t i, const int32_t n) {
+__device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t i) {
     bool cont = false, shadow = false;
     int32_t p = 0, root = 0;
     tt_ray nr{}, sr{};
@@ -1118,7 +1144,7 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
     const SceneView &sv = a.sv;
     const float p_env = sv.env ? (sv.num_emit > 0 ? 0.5f : 1.0f) : 0.0f;
     const float p_emit = sv.num_emit > 0 ? 1.0f - p_env : 0.0f;
-    if (i < n) {
+    if (i >= 0) {
         // the camera bounce's state is the generated one: path p in slot p, throughput 1,
         // roulette weight 1
         const bool first = a.bounce == 0;
@@ -1180,10 +1206,14 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
                 // the same rule, so their rows were inferred)
                 const bool guided = GUIDED && a.gd.raw != nullptr && guide_eligible(m, a.gd.min_rough);
                 Mixture lobes;
-                if (guided) decode_mixture(a.gd.raw + (int64_t)i * kGuideNOutPad16, lobes);
+                // rows of the network follow the queue's sequence
+                const int64_t row = !GUIDED || !a.queue.seg
+                                        ? i
+                                        : position_of((int)(blockIdx.x % kSegs), i - (int32_t)(blockIdx.x % kSegs) * a.queue.seg);
+                if (guided) decode_mixture(a.gd.raw + row * kGuideNOutPad16, lobes);
                 const float alpha = !guided ? 0.0f
                                             : a.gd.learn_alpha
-                                                  ? learned_alpha(a.gd.raw[(int64_t)i * kGuideNOutPad16 + kGuideAlphaOut])
+                                                  ? learned_alpha(a.gd.raw[row * kGuideNOutPad16 + kGuideAlphaOut])
                                                   : a.gd.alpha;
                 // next-event estimation
                 if (!smooth && (p_env > 0.0f || p_emit > 0.0f) && wol.z > 0.0f) {
@@ -1328,7 +1358,10 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
         if (GUIDED || first || adds) a.L[p] = Ls;
     }
     int slot, sslot;
-    block_append2(cont, &a.counts[a.nxt], shadow, &a.counts[a.scount], &slot, &sslot);
+    const int s = (int)(blockIdx.x % kSegs);
+    block_append2(cont, &a.out_counts[s * kSegStride], shadow, &a.sh_counts[s * kSegStride], &slot, &sslot);
+    slot += s * a.seg;
+    sslot += s * a.seg;
     if (cont) {
         a.rays_out[slot] = nr;
         a.thr_out[slot] = nthr;
@@ -1345,14 +1378,13 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
 // as k_shade_reference: one thread per slot, empty blocks leave at once
 template <bool GUIDED>
 __global__ __launch_bounds__(kAppendBlock) void k_shade_path(ShadeArgs a) {
-    const int32_t n = a.counts[a.cur];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.stats[0], (unsigned long long)n);
-    if ((int64_t)blockIdx.x * kAppendBlock >= n) return;
-    shade_path_one<GUIDED>(a, (int32_t)(blockIdx.x * kAppendBlock + threadIdx.x), n);
+    int32_t first, n;
+    if (!shade_block(a, &first, &n)) return;
+    shade_path_one<GUIDED>(a, (int32_t)threadIdx.x < n ? first + (int32_t)threadIdx.x : -1);
 }
 
 struct ApplyArgs {
-    const int32_t *n_dev;   // the bounce's next-event queue length
+    Queue queue;            // the bounce's next-event queue
     const int32_t *occ;
     const float4 *contrib;
     float4 *Lsh;         // per-path next-event radiance in xyz
@@ -1362,10 +1394,11 @@ struct ApplyArgs {
 };
 
 __global__ __launch_bounds__(256) void k_apply_shadow(ApplyArgs a) {
-    const int32_t n = *a.n_dev;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.stats[1], (unsigned long long)n);
-    for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (a.occ[i]) continue;
+    const int32_t n = queue_span(a.queue);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.stats[1], (unsigned long long)queue_total(a.queue));
+    for (int32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int32_t i = queue_slot(a.queue, k);
+        if (i < 0 || a.occ[i]) continue;
         const float4 c = a.contrib[i];
         const int32_t path = __float_as_int(c.w);
         const int tc = train_slot(a.gd, path);
@@ -1758,7 +1791,15 @@ struct GuideRun {
     float first_loss = 0.0f;  // loss of the first Adam step
 };
 
+// Entries of a segment: whatever its blocks can append, one each for every slot they shade
+// (block b of the camera rays and block b / kSegs of segment b % kSegs append to b % kSegs).
+int32_t segment_cap(int32_t cap) {
+    const int32_t blocks = (int32_t)(((int64_t)cap + kAppendBlock - 1) / kAppendBlock);
+    return (blocks + kSegs - 1) / kSegs * kAppendBlock;
+}
+
 tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64, bool roots) {
+    const int32_t slots = kSegs * segment_cap(cap);
     RenderState *rs = s->rs;
     if (rs && rs->cap >= cap && rs->pix_cap >= npix && (!fp64 || rs->acc64_cap >= npix) && (!roots || rs->roots))
         return TT_OK;
@@ -1774,21 +1815,21 @@ tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64, bool r
         if (st == TT_OK) st = dev_alloc(s->ctx, p, bytes, what);
     };
     for (int k = 0; k < 2; ++k) {
-        al((void **)&rs->rays[k], (size_t)cap * sizeof(tt_ray), "render rays");
-        al((void **)&rs->path[k], (size_t)cap * 4, "render path ids");
-        if (roots) al((void **)&rs->root[k], (size_t)cap * 4, "render ray roots");
-        al((void **)&rs->thr[k], (size_t)cap * 16, "render throughput");
+        al((void **)&rs->rays[k], (size_t)slots * sizeof(tt_ray), "render rays");
+        al((void **)&rs->path[k], (size_t)slots * 4, "render path ids");
+        if (roots) al((void **)&rs->root[k], (size_t)slots * 4, "render ray roots");
+        al((void **)&rs->thr[k], (size_t)slots * 16, "render throughput");
     }
-    al((void **)&rs->hits, (size_t)cap * sizeof(tt_hit), "render hits");
+    al((void **)&rs->hits, (size_t)slots * sizeof(tt_hit), "render hits");
     al((void **)&rs->L, (size_t)cap * 16, "render radiance");
     al((void **)&rs->Lsh, (size_t)cap * 16, "render next-event radiance");
     for (int k = 0; k < 2; ++k) {
-        al((void **)&rs->srays[k], (size_t)cap * sizeof(tt_ray), "render shadow rays");
-        if (roots) al((void **)&rs->sroot[k], (size_t)cap * 4, "render shadow roots");
-        al((void **)&rs->scontrib[k], (size_t)cap * 16, "render shadow contributions");
-        al((void **)&rs->socc[k], (size_t)cap * 4, "render shadow flags");
+        al((void **)&rs->srays[k], (size_t)slots * sizeof(tt_ray), "render shadow rays");
+        if (roots) al((void **)&rs->sroot[k], (size_t)slots * 4, "render shadow roots");
+        al((void **)&rs->scontrib[k], (size_t)slots * 16, "render shadow contributions");
+        al((void **)&rs->socc[k], (size_t)slots * 4, "render shadow flags");
     }
-    al((void **)&rs->counts, 32, "render queue counts");
+    al((void **)&rs->counts, (kCameraCount + 1) * 4, "render queue counts");
     al((void **)&rs->stats, 16, "render stats");
     al((void **)&rs->sample_dev, 16, "render sample index");
     al((void **)&rs->table, sizeof(SceneTable), "render scene table");
@@ -1808,7 +1849,7 @@ tt_status ensure_state(tt_scene *s, int32_t cap, int32_t npix, bool fp64, bool r
 // buffers alternate by bounce (set b & 1), and the apply adds into the paths' own
 // next-event radiance (Lsh, summed with L at the end of the pass) and credits training
 // records in fields of their own, so a shade kernel waits only for the next-event work
-// two bounces back, the last user of its set. The queue length of bounce b is counts[2 + (b & 3)]: the extension trace zeroes the one
+// two bounces back, the last user of its set. Bounce b's is queue 2 + (b & 3): the extension trace zeroes the counters
 // its shade kernel appends to, three bounces past the last next-event work that read
 // it, which a shade kernel before it has waited for. Small late-bounce queues leave
 // most of the GPU idle behind their slowest rays; the launches fill it together.
@@ -1825,16 +1866,21 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     // the small queue kernels stride over the device-side count with 16 blocks of 256
     // threads per CU; the shade kernels take one thread per slot of the capacity
     static_assert(kAppendBlock == 256, "shade launches use the 256-thread grid");
+    const int32_t seg = segment_cap(cap), slots = kSegs * seg;
     const unsigned gblocks =
         (unsigned)std::min<int64_t>(((int64_t)cap + 255) / 256, 16LL * std::max(1, s->ctx->num_cus));
-    const unsigned sblocks = (unsigned)(((int64_t)cap + kAppendBlock - 1) / kAppendBlock);
+    const unsigned sblocks = (unsigned)(slots / kAppendBlock);
+    // the camera rays are one run
+    const Queue in{rs->counts + (b == 0 ? kCameraCount : cur * kQueue), b == 0 ? 0 : seg};
+    const Queue events{rs->counts + sc * kQueue, seg};
     TraceArgs ta = trace_args(s);
     ta.rays = rs->rays[cur];
     ta.hits = rs->hits;
-    ta.n = cap;
-    ta.n_dev = rs->counts + cur;
-    ta.reset0 = rs->counts + nxt;
-    ta.reset1 = rs->counts + sc;
+    ta.n = b == 0 ? cap : slots;
+    ta.n_dev = in.counts;
+    ta.seg = in.seg;
+    ta.reset0 = rs->counts + nxt * kQueue;
+    ta.reset1 = rs->counts + sc * kQueue;
     ta.ray_root = rs->root[cur];
     // camera rays (bounce 0) are coherent and their queue is full: one wave per
     // 64-ray group; later extension and shadow queues: persistent waves that refill once
@@ -1846,7 +1892,7 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     hipError_t e = launch_trace(ta, variant, false, lds, block, 0, refill_ext, s->ctx->num_cus, hs, tri_mode);
     if (e != hipSuccess) return e;
     if (sv.num_geoms > 0) {
-        GeomArgs ga{rs->rays[cur], rs->hits, nullptr, rs->counts + cur, sv.geoms, sv.num_geoms};
+        GeomArgs ga{rs->rays[cur], rs->hits, nullptr, in, sv.geoms, sv.num_geoms};
         hipLaunchKernelGGL(k_geom_hits, dim3(gblocks), dim3(256), 0, hs, ga);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -1860,13 +1906,13 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
         // guide inference over the hit queue: inputs, flags and counts, the guided slots
         // in slot order, then the MLP over that list
         tt_guide *g = gr->g;
-        if ((int64_t)cap > g->icap) return hipErrorInvalidValue;   // the inference rows cover the queue
-        const unsigned rblocks = (unsigned)std::min<int64_t>(((int64_t)cap + 255) / 256, g->iblocks);
+        if ((int64_t)slots > g->icap) return hipErrorInvalidValue;   // the inference rows cover the queue
+        const unsigned rblocks = (unsigned)std::min<int64_t>(slots / 256, g->iblocks);
         int32_t *rows_dev = g->iblock_n + g->iblocks;
-        GuideInArgs ga{gr->gd, sv, rs->rays[cur], rs->hits, rs->counts, cur, g->iin, g->imask, g->iblock_n, nullptr};
+        GuideInArgs ga{gr->gd, sv, rs->rays[cur], rs->hits, in, g->iin, g->imask, g->iblock_n, nullptr};
         hipLaunchKernelGGL(k_guide_inputs<false>, dim3(rblocks), dim3(256), 0, hs, ga);
         hipLaunchKernelGGL(k_guide_slots, dim3(rblocks), dim3(256), 0, hs, (const uint64_t *)g->imask,
-                           (const int32_t *)g->iblock_n, rs->counts + cur, g->islot, rows_dev);
+                           (const int32_t *)g->iblock_n, in, g->islot, rows_dev);
         e = hipGetLastError();
         if (e == hipSuccess) e = guide_infer(g, g->iin, g->iraw, cap, rows_dev, hs, g->islot);
         if (e != hipSuccess) return e;
@@ -1891,10 +1937,10 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     sa.thr_out = rs->thr[nxt];
     sa.L = rs->L;
     sa.Lsh = rs->Lsh;
-    sa.counts = rs->counts;
-    sa.cur = cur;
-    sa.nxt = nxt;
-    sa.scount = sc;
+    sa.queue = in;
+    sa.out_counts = rs->counts + nxt * kQueue;
+    sa.sh_counts = rs->counts + sc * kQueue;
+    sa.seg = seg;
     sa.srays = rs->srays[set];
     sa.scontrib = rs->scontrib[set];
     sa.acc = rs->acc;
@@ -1926,18 +1972,19 @@ hipError_t launch_bounce(tt_scene *s, RenderState *rs, const tt_render_params *p
     TraceArgs sh = trace_args(s);
     sh.rays = rs->srays[set];
     sh.flags = rs->socc[set];
-    sh.n = cap;
-    sh.n_dev = rs->counts + sc;
+    sh.n = slots;
+    sh.n_dev = events.counts;
+    sh.seg = seg;
     sh.ray_root = rs->sroot[set];
     e = launch_trace(sh, variant, true, lds, block, 0, refill_later, s->ctx->num_cus, ss, kTriTwoSided);
     if (e != hipSuccess) return e;
     if (sv.num_geoms > 0) {
-        GeomArgs go{rs->srays[set], nullptr, rs->socc[set], rs->counts + sc, sv.geoms, sv.num_geoms};
+        GeomArgs go{rs->srays[set], nullptr, rs->socc[set], events, sv.geoms, sv.num_geoms};
         hipLaunchKernelGGL(k_geom_occluded, dim3(gblocks), dim3(256), 0, ss, go);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    ApplyArgs aa{rs->counts + sc, rs->socc[set], rs->scontrib[set], rs->Lsh, rs->stats, b, p->max_depth,
+    ApplyArgs aa{events, rs->socc[set], rs->scontrib[set], rs->Lsh, rs->stats, b, p->max_depth,
                  gr ? gr->gd : GuideShade{}};
     hipLaunchKernelGGL(k_apply_shadow, dim3(gblocks), dim3(256), 0, ss, aa);
     e = hipGetLastError();
@@ -2171,7 +2218,7 @@ tt_status render_impl(tt_scene *s, int32_t nsc, const tt_camera *cams, const tt_
     hipStream_t hs = ctx->stream;
     if (gr) {
         // inference rows: one per queued path; training rows: batch_rows
-        st = guide_alloc_infer(gr->g, (int64_t)npix * k_after);
+        st = guide_alloc_infer(gr->g, kSegs * (int64_t)segment_cap(npix * k_after));
         if (st == TT_OK && gr->train) st = guide_alloc_batch(gr->g, gr->batch_rows);
         if (st == TT_OK && gr->train) {
             const int32_t want = std::max(1, gr->gd.ntrain);
@@ -2622,15 +2669,14 @@ tt_status tt_debug_guide_infer_slots(tt_guide *g, const float *inputs, const int
     if (e == hipSuccess) {
         const unsigned rblocks = (unsigned)std::min<int64_t>((n + 255) / 256, g->iblocks);
         GuideInArgs ga{};
-        ga.counts = d_n;
-        ga.cur = 0;
+        ga.queue = Queue{d_n, 0};
         ga.in = g->iin;
         ga.mask = g->imask;
         ga.block_n = g->iblock_n;
         ga.given = d_given;
         hipLaunchKernelGGL(k_guide_inputs<true>, dim3(rblocks), dim3(256), 0, hs, ga);
         hipLaunchKernelGGL(k_guide_slots, dim3(rblocks), dim3(256), 0, hs, (const uint64_t *)g->imask,
-                           (const int32_t *)g->iblock_n, (const int32_t *)d_n, g->islot, rows_dev);
+                           (const int32_t *)g->iblock_n, ga.queue, g->islot, rows_dev);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = guide_infer(g, g->iin, g->iraw, n, rows_dev, hs, g->islot);

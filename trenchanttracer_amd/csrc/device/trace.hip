@@ -283,6 +283,32 @@ __device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, 
     return false;
 }
 
+// The counts of the queue traced, uniform, and the slot of its r-th position (-1: none).
+struct SegmentCounts {
+    int32_t n0 = 0, n1 = 0, n2 = 0, n3 = 0;   // (an array would go to scratch memory)
+    static_assert(kSegs == 4, "one count each");
+    __device__ __forceinline__ int32_t read(const TraceArgs &a) {
+        n0 = __builtin_amdgcn_readfirstlane(*a.n_dev);
+        if (!a.seg) return n0;
+        n1 = __builtin_amdgcn_readfirstlane(a.n_dev[kSegStride]);
+        n2 = __builtin_amdgcn_readfirstlane(a.n_dev[2 * kSegStride]);
+        n3 = __builtin_amdgcn_readfirstlane(a.n_dev[3 * kSegStride]);
+        return (max(max(n0, n1), max(n2, n3)) + 63) / 64 * (64 * kSegs);
+    }
+    __device__ __forceinline__ int32_t slot(const TraceArgs &a, int32_t r) const {
+        if (!a.seg) return r;
+        const int s = segment_of(r);
+        const int32_t i = entry_of(r), lo = s & 1 ? n1 : n0, hi = s & 1 ? n3 : n2;
+        return i < (s & 2 ? hi : lo) ? s * a.seg + i : -1;
+    }
+};
+__device__ __forceinline__ void reset_counts(const TraceArgs &a, int tid) {
+    if (blockIdx.x == 0 && tid < kSegs) {
+        if (a.reset0) a.reset0[tid * kSegStride] = 0;
+        if (a.reset1) a.reset1[tid * kSegStride] = 0;
+    }
+}
+
 // log2 of the rays of a group (TraceArgs::spread), uniform.
 __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
     if (!spread || n == 0u) return 6;
@@ -313,11 +339,9 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
         if (vb < (q << 3)) vb = (vb & 7u) * q + (vb >> 3);
     }
     uint32_t n = (uint32_t)a.n;   // below 2^31 (launch_trace)
-    if (a.n_dev) n = min((uint32_t)max(0, *a.n_dev), n);
-    if (blockIdx.x == 0 && tid == 0) {
-        if (a.reset0) *a.reset0 = 0;
-        if (a.reset1) *a.reset1 = 0;
-    }
+    SegmentCounts in;
+    if (a.n_dev) n = min((uint32_t)max(0, in.read(a)), n);
+    reset_counts(a, tid);
     // Launch forms. One wave per 64-ray group; persistent waves (Aila & Laine's persistent
     // threads with ray replacement): the grid holds about as many waves as the chip keeps
     // resident, and wave w of W owns the groups w, w + W, w + 2W, ... in that order, so that
@@ -400,7 +424,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
             const uint32_t q = cursor + (uint32_t)__popcll(m & below);
             if (q < total) {
                 const uint32_t r = (((q >> gs) * waves + first) << gs) + (q & ((1u << gs) - 1u));
-                if (r < n) rid = (int)(a.order ? a.order[r] : r);
+                if (r < n) rid = a.order ? (int)a.order[r] : in.slot(a, (int)r);
             }
             if (rid >= 0) {
                 const float4 *rp = reinterpret_cast<const float4 *>(a.rays + rid);
@@ -593,11 +617,9 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
         if (vb < (q << 3)) vb = (vb & 7u) * q + (vb >> 3);
     }
     int64_t n = a.n;
-    if (a.n_dev) n = min((int64_t)*a.n_dev, n);
-    if (blockIdx.x == 0 && tid == 0) {
-        if (a.reset0) *a.reset0 = 0;
-        if (a.reset1) *a.reset1 = 0;
-    }
+    SegmentCounts in;
+    if (a.n_dev) n = min((int64_t)in.read(a), n);
+    reset_counts(a, tid);
     // the launch form of k_trace_wide
     const int gs = group_bits((uint32_t)max((int64_t)0, n), a.spread);
     const int64_t groups = (n + (1 << gs) - 1) >> gs;
@@ -656,7 +678,7 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs a) {
             const int64_t q = cursor + __popcll(m & below);
             if (q < total) {
                 const int64_t r = (((q >> gs) * waves + w) << gs) + (q & ((1 << gs) - 1));
-                if (r < n) rid = a.order ? (int64_t)a.order[r] : r;
+                if (r < n) rid = a.order ? (int64_t)a.order[r] : in.slot(a, (int)r);
             }
             if (rid >= 0) {
                 const float4 *rp = reinterpret_cast<const float4 *>(a.rays + rid);
