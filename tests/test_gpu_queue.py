@@ -42,3 +42,25 @@ def test_path_render_does_not_depend_on_the_passes(tt, ctx, w, h, spp):
     for got in out[1:]:
         assert np.array_equal(got[0], out[0][0]) and got[1:] == out[0][1:]
     scene.close()
+
+
+@pytest.mark.parametrize("spp", [1, 8, 9, 16, 17, 32, 33, 70])
+def test_sample_sums_match_oracle_and_passes(tt, oracle, ctx, spp):
+    """Samples per pass around the chunks a block of pixels is summed in, on pixel counts
+    that leave a partial block."""
+    from trenchanttracer_amd import workloads
+    print(f"sample sums: {spp} samples", file=sys.stderr, flush=True)
+    for w, h in ((9, 8), (29, 9)):
+        mesh, mats, cam = workloads.cornell(subdiv=1, width=w, height=h)
+        bvh = tt.BVH.build(mesh)
+        scene = tt.DeviceScene(ctx, mesh, bvh, mats)
+        img, _ = scene.render(cam, tt.render_params(spp=spp, max_depth=4, seed=6, mode=tt.RENDER_REFERENCE))
+        want = oracle.render_ref(oracle.CompactBVH(bvh.export_compact()), mesh.arrays(), mats, cam, spp=spp,
+                                 max_depth=4, seed=6, env=None)
+        assert np.array_equal(img.view(np.int32), want.view(np.int32))
+        prm = dict(spp=spp, max_depth=4, rr_depth=2, seed=7, mode=tt.RENDER_PATH)
+        for fp64 in (False, True):
+            a = scene.render(cam, tt.render_params(fp64=fp64, **prm))[0]
+            b = scene.render(cam, tt.render_params(fp64=fp64, paths_in_flight=w * h, **prm))[0]
+            assert np.array_equal(a.view(np.int32), b.view(np.int32)) and a.max() > 0
+        scene.close()

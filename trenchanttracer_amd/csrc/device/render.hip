@@ -1431,41 +1431,49 @@ __device__ __forceinline__ int32_t slot_pixel(const SceneTable *t, int32_t q) {
     return t->pix_off[sid] + local;
 }
 
-// A block's 256 slots have their samples side by side (path ids q * kk + s); the
-// block stages them in LDS kResolveChunk samples at a time, each pixel's chunk read
-// as one 128-byte segment (a thread per slot reading its own samples would put the
-// wave's 64 loads 16 * kk bytes apart). Rows are padded to kResolveChunk + 1 float4
-// so that both the staging writes and each thread's row reads hit distinct banks.
-constexpr int kResolveChunk = 8;
+// A block's P slots have their samples side by side (path ids q * kk + s); the block stages
+// them in LDS 2048 / P samples at a time, each pixel's chunk read as one run (a thread per
+// slot reading its own samples would put the wave's 64 loads 16 * kk bytes apart), and P
+// threads add them, one per pixel. Rows are padded by a float4 so that both the staging
+// writes and each thread's row reads hit distinct banks.
+// Bound by HBM in large renders, by latency in small ones: a 256 x 256 image has one block of
+// 256 slots per CU, four of 64. So P is the smallest whose chunk a pass's samples fill (2048
+// loads in flight per block): with 256 / 64 slots, 64 samples of 256 x 256 51 / 30 us, of 1080p
+// 745 / 683, but 16 samples of a batch 124 / 146 and one sample of 640 x 360 5.8 / 7.9.
+template <int P>
 struct ResolveTile {
-    float4 v[256][kResolveChunk + 1];
+    static constexpr int kChunk = 2048 / P;
+    float4 v[P][kChunk + 1];
 };
+int resolve_pixels(int32_t kk) { return kk <= 8 ? 256 : kk <= 16 ? 128 : 64; }
 
 // Lsh (path mode): each path's next-event radiance, added to its other radiance (yzw).
-__device__ __forceinline__ void stage_chunk(ResolveTile &t, const float4 *L, const float4 *Lsh, int32_t q0,
-                                            int32_t npix, int32_t kk, int32_t s0) {
-    for (int i = threadIdx.x; i < 256 * kResolveChunk; i += 256) {
-        const int pl = i / kResolveChunk, j = i - pl * kResolveChunk;
-        const int32_t q = q0 + pl, s = s0 + j;
-        if (q < npix && s < kk) {
-            const int32_t id = path_id(q, s, kk);
-            float4 v = L[id];
-            if (Lsh) {
-                const float4 e = Lsh[id];
-                v.y += e.x;
-                v.z += e.y;
-                v.w += e.z;
-            }
-            t.v[pl][j] = v;
+// m: samples of the chunk.
+template <int P>
+__device__ __forceinline__ void stage_chunk(ResolveTile<P> &t, const float4 *L, const float4 *Lsh, int32_t q0,
+                                            int32_t npix, int32_t kk, int32_t s0, int32_t m) {
+    const int32_t n = min(P, npix - q0) * m;
+    const float inv = 1.0f / (float)m;
+    for (int i = threadIdx.x; i < n; i += 256) {
+        const int pl = (int)(((float)i + 0.5f) * inv), j = i - pl * m;   // i / m, i below 2048
+        const int32_t id = path_id(q0 + pl, s0 + j, kk);
+        float4 v = L[id];
+        if (Lsh) {
+            const float4 e = Lsh[id];
+            v.y += e.x;
+            v.z += e.y;
+            v.w += e.z;
         }
+        t.v[pl][j] = v;
     }
 }
 
+template <int P>
 __global__ __launch_bounds__(256) void k_resolve_reference(const SceneTable *tab, const float4 *L, int32_t npix,
                                                            int32_t kk, float inv_spp, float *acc) {
-    __shared__ ResolveTile t;
-    const int32_t q0 = blockIdx.x * 256, q = q0 + threadIdx.x;
-    const bool live = q < npix;
+    __shared__ ResolveTile<P> t;
+    const int32_t q0 = blockIdx.x * P, q = q0 + threadIdx.x;
+    const bool live = threadIdx.x < P && q < npix;
     float *o = acc + 3 * (int64_t)(live ? slot_pixel(tab, q) : 0);
     float r = 0.0f, g = 0.0f, b = 0.0f;
     if (live) {
@@ -1473,12 +1481,12 @@ __global__ __launch_bounds__(256) void k_resolve_reference(const SceneTable *tab
         g = o[1];
         b = o[2];
     }
-    for (int32_t s0 = 0; s0 < kk; s0 += kResolveChunk) {
+    for (int32_t s0 = 0; s0 < kk; s0 += t.kChunk) {
         __syncthreads();
-        stage_chunk(t, L, nullptr, q0, npix, kk, s0);
+        const int32_t m = min(t.kChunk, kk - s0);
+        stage_chunk(t, L, nullptr, q0, npix, kk, s0, m);
         __syncthreads();
-        const int32_t m = min(kResolveChunk, kk - s0);
-        for (int j = 0; j < m; ++j) {
+        for (int j = 0; live && j < m; ++j) {
             const float4 v = t.v[threadIdx.x][j];
             r = r + v.x * inv_spp;
             g = g + v.y * inv_spp;
@@ -1497,11 +1505,12 @@ __global__ __launch_bounds__(256) void k_resolve_reference(const SceneTable *tab
 // the sum is the same left fold over the pixel's samples for any pass structure
 // (a batch of scenes, whose passes split the samples differently, gives each scene
 // the bits of its own render).
+template <int P>
 __global__ __launch_bounds__(256) void k_resolve(const SceneTable *tab, const float4 *L, const float4 *Lsh,
                                                  int32_t npix, int32_t kk, float *acc, double *acc64) {
-    __shared__ ResolveTile t;
-    const int32_t q0 = blockIdx.x * 256, q = q0 + threadIdx.x;
-    const bool live = q < npix;
+    __shared__ ResolveTile<P> t;
+    const int32_t q0 = blockIdx.x * P, q = q0 + threadIdx.x;
+    const bool live = threadIdx.x < P && q < npix;
     const int32_t pix = live ? slot_pixel(tab, q) : 0;
     double rd = 0.0, gd = 0.0, bd = 0.0;
     float rf = 0.0f, gf = 0.0f, bf = 0.0f;
@@ -1518,12 +1527,12 @@ __global__ __launch_bounds__(256) void k_resolve(const SceneTable *tab, const fl
             bf = o[2];
         }
     }
-    for (int32_t s0 = 0; s0 < kk; s0 += kResolveChunk) {
+    for (int32_t s0 = 0; s0 < kk; s0 += t.kChunk) {
         __syncthreads();
-        stage_chunk(t, L, Lsh, q0, npix, kk, s0);
+        const int32_t m = min(t.kChunk, kk - s0);
+        stage_chunk(t, L, Lsh, q0, npix, kk, s0, m);
         __syncthreads();
-        const int32_t m = min(kResolveChunk, kk - s0);
-        for (int j = 0; j < m; ++j) {
+        for (int j = 0; live && j < m; ++j) {
             const float4 v = t.v[threadIdx.x][j];
             if (acc64) {
                 rd += (double)v.y;
@@ -2026,13 +2035,17 @@ hipError_t launch_pass(tt_scene *s, RenderState *rs, const tt_render_params *p, 
         const hipError_t j = hipStreamWaitEvent(hs, s->ctx->shadow_done[(p->max_depth - 1) & 1], 0);
         if (e == hipSuccess) e = j;
     }
+    const int P = resolve_pixels(kk);
     if (e == hipSuccess && p->mode == TT_RENDER_PATH) {
-        hipLaunchKernelGGL(k_resolve, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, hs, g.tab,
+        const auto kernel = P == 256 ? k_resolve<256> : P == 128 ? k_resolve<128> : k_resolve<64>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((npix + P - 1) / P)), dim3(256), 0, hs, g.tab,
                            (const float4 *)rs->L, (const float4 *)rs->Lsh, npix, kk, fp64 ? nullptr : rs->acc,
                            fp64 ? rs->acc64 : nullptr);
         e = hipGetLastError();
     } else if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_resolve_reference, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, hs, g.tab,
+        const auto kernel =
+            P == 256 ? k_resolve_reference<256> : P == 128 ? k_resolve_reference<128> : k_resolve_reference<64>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((npix + P - 1) / P)), dim3(256), 0, hs, g.tab,
                            (const float4 *)rs->L, npix, kk, 1.0f / (float)p->spp, rs->acc);
         e = hipGetLastError();
     }
