@@ -1136,8 +1136,11 @@ __global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const
 // for the traversal only when there are several, and the camera bounce's path ids are not
 // stored. Against state by path id, read and written on every bounce: 33.0 -> 29.1 ms of
 // shading in the 1080p, 64 spp, depth 16 render over 1.3M triangles (103.6 -> 99.6 ms,
-// traced), 76 VGPRs against 84. Gathering a block's hits before its misses, for fuller
+// traced). Gathering a block's hits before its misses, for fuller
 // waves, gave nothing (33.2 -> 33.8 ms).
+// Registers are held to 72 (7 waves per SIMD; guided 128, 4 waves, 2 spilled): room
+// 1731 -> 1698 us, batch 12.27 -> 12.15 ms, 1080p 92.2 -> 91.9; guided (135 before) 12.59 ->
+// 12.43 ms. 8 waves spill: room 2048 us.
 template <bool GUIDED>
 __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t i) {
     bool cont = false, shadow = false;
@@ -1381,7 +1384,7 @@ __device__ __forceinline__ void shade_path_one(const ShadeArgs &a, const int32_t
 
 // as k_shade_reference: one thread per slot, empty blocks leave at once
 template <bool GUIDED>
-__global__ __launch_bounds__(kAppendBlock) void k_shade_path(ShadeArgs a) {
+__global__ __launch_bounds__(kAppendBlock, GUIDED ? 4 : 7) void k_shade_path(ShadeArgs a) {
     int32_t first, n;
     if (!shade_block(a, &first, &n)) return;
     shade_path_one<GUIDED>(a, (int32_t)threadIdx.x < n ? first + (int32_t)threadIdx.x : -1);
