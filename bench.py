@@ -131,7 +131,7 @@ def main():
         d_hh.free()
     log(f"halves: {halves}")
 
-    # the traversal's own loop replayed without its box and triangle arithmetic, in
+    # the two-child traversal loop replayed without its box and triangle arithmetic, in
     # the headline's launch form, after the same key pass and sort
     # (tt_bench_fetch_replay); the whole set and each half
     # (the exact loop's counting launch gives the algorithmic bytes: its node visits
@@ -340,9 +340,10 @@ def pmc_call_traffic(args, timeout=240):
         copy = [v for k, v in rows if "k_copy16" in k]
         gather = [v for k, v in rows if "k_gather64" in k]
         # the call: its dispatches up to its traversal launch (the buffer fills after
-        # it belong to the gather probe and the copy)
+        # it belong to the gather probe and the copy), past the scene's creation
         last = max((i for i, (k, _) in enumerate(rows) if "k_trace" in k), default=-1)
-        call = rows[:last + 1]
+        first = max((i for i, (k, _) in enumerate(rows[:last + 1]) if "k_wide" in k), default=-1) + 1
+        call = rows[first:last + 1]
         if len(copy) != 1 or len(gather) != 1 or not call:
             return None, f"{counter}: unexpected dispatches {[k for k, _ in rows]}"
         kib[counter] = (copy[0], call, gather[0])
@@ -378,18 +379,18 @@ def host_cpu():
 
 def committed_traffic(args):
     """The counter profile committed for the headline configuration
-    (profiles/k_trace_speculative_soup1M_pmc.md), used only when the live counter runs
+    (profiles/k_trace_wide_soup1M_pmc.md), used only when the live counter runs
     cannot run; None for any other configuration."""
     if (args.variant, args.lds_stack, args.block, args.refill, args.reorder, args.ntris) != (1, 16, 256, 32, 1,
                                                                                           1_000_000):
         return None, "no live counter runs and no committed profile for this configuration"
-    sr = 262_144 / 131_079.5
+    sr = 262_144 / 131_079.4
     # keys, 3 scans, 3 scatters, 2 histograms, traversal
-    fetch = 129_729.2 + 3_128.5 + 24_564.5 + 32_586.1 + 40_775.8 + 40_738.0 + 6_598_886.9
-    write = 49_932.7 + 6_120.0 + 78_975.1 + 32_480.9 + 79_058.8 + 39_029.7 + 214_054.2
-    return ({"call_bytes": (fetch * sr + write) * 1024, "trace_bytes": (6_598_886.9 * sr + 214_054.2) * 1024,
-             "gather_bytes": (4_157_602.9 * sr + 16_384.0) * 1024},
-            "profiles/k_trace_speculative_soup1M_pmc.md (committed counter runs)")
+    fetch = 129_677.4 + 3_136.5 + 24_580.1 + 32_447.0 + 40_779.9 + 40_736.9 + 5_090_486.7
+    write = 50_769.2 + 6_120.0 + 78_974.3 + 32_445.7 + 79_057.7 + 39_029.8 + 239_645.9
+    return ({"call_bytes": (fetch * sr + write) * 1024, "trace_bytes": (5_090_486.7 * sr + 239_645.9) * 1024,
+             "gather_bytes": (4_187_786.0 * sr + 16_384.0) * 1024},
+            "profiles/k_trace_wide_soup1M_pmc.md (committed counter runs)")
 
 
 def render_bench(tt, ctx, np, no_cpu):

@@ -274,7 +274,8 @@ tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double 
  * one wave per group); 1..64 = persistent waves: the launch holds as many waves as the
  * GPU keeps resident, wave w of W traces the 64-ray groups w, w + W, ..., and a lane whose
  * ray is done takes the wave's next ray once at least `refill` of its 64 lanes are idle
- * (keeps incoherent waves full; sweeps take rays at 32).
+ * (keeps incoherent waves full; sweeps take rays at 32). With fewer than 64 rays for each
+ * of 8 waves per CU the groups are smaller, in every form.
  * xcd_order: 0 = waves in launch order; 1 = blocks are renumbered so that each of the
  * 8 XCDs (which take blocks round-robin) holds one contiguous range of waves.
  * reorder: 0 (default) = rays are traced in the caller's order; 1 = the call first
@@ -322,8 +323,8 @@ tt_status tt_trace_any(tt_scene *s, const tt_ray *rays, int64_t n, int32_t *hit_
 tt_status tt_trace_closest_noalloc(tt_scene *s, const tt_ray *rays, int64_t n, tt_hit *hits,
                                    const tt_trace_cfg *cfg, void *stream);
 /* Node-fetch roofline probe for a ray set (no reference counterpart): the time of
- * the traversal's own loop without its arithmetic. A recording launch of the
- * closest-hit loop (cfg->variant, LDS stack 16, cfg's block / refill / reorder) stores
+ * the two-child loop without its arithmetic, over scenes of every kind. A recording launch
+ * of the closest-hit loop (cfg->variant, LDS stack 16, cfg's block / refill / reorder) stores
  * the outcome of every node's slab test (4 bits: which children are entered, in which
  * order); the replay launch then runs the same loop over the same rays in the same
  * launch form (same waves, stack, leaf postponement, ballots and refills) with each

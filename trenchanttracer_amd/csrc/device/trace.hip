@@ -321,7 +321,7 @@ __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
 // issue 90% and the address path 82% busy, with 32% of the lanes active: 1.85e9 VALU
 // instructions, 1.53e9 cache accesses and 4.0 ms a launch. Visiting four boxes with 3 loads
 // instead of 8, and taking node visits and triangle tests by the vote below (59% of the
-// lanes active), takes 1.45e9, 1.04e9 and 3.0 ms; each alone gains little, as the other
+// lanes active), takes 1.43e9, 0.90e9 and 3.0 ms; each alone gains little, as the other
 // limit holds (four children in the while-while loop: 6.6 ms, slower).
 template <bool ANY, int S, int TRI>
 __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {

@@ -46,7 +46,7 @@ def main():
     ap.add_argument("--variant", type=int, default=1)
     ap.add_argument("--lds-stack", type=int, default=16)
     ap.add_argument("--block", type=int, default=64)
-    ap.add_argument("--refill", type=int, default=0, help="traversal: refill threshold (0: one wave per group)")
+    ap.add_argument("--refill", type=int, default=0, help="traversal: refill threshold (0: sweeps over the range)")
     ap.add_argument("--reorder", type=int, default=0, help="traversal: 1 = trace in Morton order of the origins")
     ap.add_argument("--case", choices=("traversal", "pathtrace", "train", "guided"), default="traversal")
     ap.add_argument("--paths-in-flight", type=int, default=0, help="pathtrace: paths per pass (0: the default)")
