@@ -28,7 +28,11 @@
 // cover (non-finite or overflowing terms, negative tmin, a full stack), the lane walks the
 // two-child tree. An any-hit ray applies the leaf test to every triangle it would accept.
 // (Boxes are culled against the best distance with 2^-10 to spare: a triangle whose
-// computed t lies further than that below its own box could still be skipped.)
+// computed t lies further than that below its own box could still be skipped. That takes
+// |det| near the 1e-5 it is accepted from and edges whose product is large against it: of
+// 5M rays aimed within 1e-8 to 1e-2 of the planes of triangles 5 to 20 units wide, 8 got
+// another hit than the single-lane order's, which were at distances such as 4.0 for a
+// triangle 11.8 away. A margin of 2^-6 finds no more of them and costs 1.5 to 4%.)
 //
 // Stack: the lowest S entries of each lane live in LDS ([entry][lane] so the lanes of a
 // wave hit distinct banks), deeper entries in per-lane scratch.
