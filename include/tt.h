@@ -270,7 +270,8 @@ tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double 
  * too, but for triangles whose computed distance is rounding noise, more than 2^-10 below
  * their own box: of 5M rays aimed within 1e-8 to 1e-2 of the planes of triangles 5 to 20
  * units wide, 8 records differ (the speculative loop: 4; rays not aimed so: none of 400M).
- * lds_stack: LDS stack entries of 4 bytes per
+ * Closest-hit calls of variant 0 therefore keep the two-child loop on scenes with a
+ * triangle whose edges' lengths multiply to more than 1. lds_stack: LDS stack entries of 4 bytes per
  * lane (8, 16, 24 or 32; a closest-hit entry of the four-child walk is 8 bytes, and 3/4 of
  * the number of them are kept in LDS); block: threads per block (64..256, multiple of 64).
  * refill: 0 (default) = the library's choice: sweeps over one part of the range after

@@ -118,7 +118,8 @@ def test_four_child_walk_matches_oracle(tt, oracle, ctx, kind):
     want, _ = cb.trace(rays)
     any_want, _ = cb.trace(rays, any_hit=True)
     hit = (oracle.hit_ids(any_want) >= 0).astype(np.int32)
-    for cfg in (None, tt.trace_cfg(0, 8, 64, refill=16), tt.trace_cfg(1, 32, 256, refill=1, reorder=1)):
+    for cfg in (None, tt.trace_cfg(0, 8, 64, refill=16), tt.trace_cfg(1, 32, 256, refill=1, reorder=1),
+                tt.trace_cfg(1, 16, 128), tt.trace_cfg(1, 8, 64, refill=16)):
         got = scene.intersect(rays, cfg)
         for k, (x, name) in enumerate(zip(got, ("id", "t", "u", "v"))):
             bad = np.flatnonzero(x.view(np.int32) != want[:, k].view(np.int32))
@@ -126,6 +127,39 @@ def test_four_child_walk_matches_oracle(tt, oracle, ctx, kind):
         flags = scene.occluded(rays, cfg)
         bad = np.flatnonzero(flags != hit)
         assert len(bad) == 0, f"{kind}: {len(bad)} flags, first ray {bad[0]}: {rays[bad[0]]}"
+    scene.close()
+
+
+@pytest.mark.parametrize("seed,tris,size", [(2, 400, 5.0), (13, 400, 20.0), (14, 100, 10.0), (15, 2000, 5.0)])
+def test_variant_0_is_exact_for_hits_of_rounding_noise(tt, oracle, ctx, seed, tris, size):
+    """Rays almost in the planes of large triangles, whose computed distances can lie far
+    from them: the records of the single-lane order."""
+    print(f"grazing rays: {tris} triangles of size {size}", file=sys.stderr, flush=True)
+    rng = np.random.default_rng(seed)
+    v = (rng.uniform(-10, 10, (tris, 1, 3)) + rng.normal(0, size, (tris, 3, 3))).astype(np.float32)
+    mesh = tt.Mesh.from_arrays(v.reshape(-1, 3), np.arange(3 * tris, dtype=np.int32).reshape(-1, 3))
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    n = 1_000_000
+    k = rng.integers(tris, size=n)
+    w = rng.dirichlet((1, 1, 1), n)
+    t = v[k].astype(np.float64)
+    p = (t * w[:, :, None]).sum(1)
+    e1, e2 = t[:, 1] - t[:, 0], t[:, 2] - t[:, 0]
+    nn = np.cross(e1, e2)
+    nn /= np.linalg.norm(nn, axis=1, keepdims=True)
+    a = rng.uniform(0, 2 * np.pi, n)
+    u = e1 / np.linalg.norm(e1, axis=1, keepdims=True)
+    off = 10 ** rng.uniform(-8, -2, n) * rng.choice([-1, 1], n)
+    d = u * np.cos(a)[:, None] + np.cross(nn, u) * np.sin(a)[:, None] + nn * off[:, None]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, :3] = p - d * (10 ** rng.uniform(-2, 1.5, n))[:, None]
+    rays[:, 4:7], rays[:, 7] = d, 1e20
+    want, _ = oracle.CompactBVH(bvh.export_compact()).trace(rays, nthreads=8)
+    for cfg in (None, tt.trace_cfg(0, 16, 256, refill=16)):
+        for j, x in enumerate(scene.intersect(rays, cfg)):
+            assert np.array_equal(x.view(np.int32), want[:, j].view(np.int32))
     scene.close()
 
 

@@ -104,6 +104,7 @@ TraceArgs trace_args(const tt_scene *s) {
     a.num_nodes = (int32_t)s->num_nodes;
     a.wide = reinterpret_cast<const uint4 *>(s->wide);
     a.wide_step = s->wide_step;
+    a.wide_size = s->wide_size;
     a.wide_bound = s->wide_bound;
     a.roots = s->roots;
     return a;

@@ -64,6 +64,7 @@ struct TraceArgs {
     int32_t num_nodes;
     const uint4 *wide;        // four-child tree and its triangle records (nullptr: walk the two-child one)
     int32_t wide_step;        // 16-byte units from one record of it to the next
+    float wide_size;          // largest |e1|^2 |e2|^2 of a triangle
     float wide_bound;         // largest coordinate of a plane
     const int32_t *ray_root;  // if set: scene of each ray (its root is that record of the wide tree)
     const int32_t *roots;     // if set: the scenes' roots in the two-child tree

@@ -41,6 +41,7 @@ struct tt_scene {
     int64_t num_tris = 0;
     void *wide = nullptr;        // the four-child tree the traversal walks, with its triangle records (wide.hip)
     int32_t wide_step = 3;       // 16-byte units from one record of it to the next
+    float wide_size = 0.0f;      // largest |e1|^2 |e2|^2 of a triangle
     float wide_bound = 0.0f;
     int32_t *roots = nullptr;    // several scenes in one tree: their two-child roots
     // shading data by original triangle id

@@ -32,7 +32,9 @@
 // |det| near the 1e-5 it is accepted from and edges whose product is large against it: of
 // 5M rays aimed within 1e-8 to 1e-2 of the planes of triangles 5 to 20 units wide, 8 got
 // another hit than the single-lane order's, which were at distances such as 4.0 for a
-// triangle 11.8 away. A margin of 2^-6 finds no more of them and costs 1.5 to 4%.)
+// triangle 11.8 away; of 3M at triangles around one unit, none. A margin of 2^-6 finds no
+// more of them and costs 1.5 to 4%. So variant 0 keeps the two-child loop where triangles
+// are that large: launch_v. The speculative loop had such misses, 4 of those 5M.)
 //
 // Stack: the lowest S entries of each lane live in LDS ([entry][lane] so the lanes of a
 // wave hit distinct banks), deeper entries in per-lane scratch.
@@ -903,7 +905,11 @@ hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int n
 // the two-child loop of the asked variant elsewhere.
 template <bool ANY, int TRI>
 hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int block, int num_cus, hipStream_t s) {
-    if (a.wide) {
+    // The exact loop is asked for and triangles are so large that the distance of one accepted
+    // at |det| > 1e-5 can be rounding noise (about 1e-2 |e1| |e2| of it): the two-child walk,
+    // as the culling of the four-child one relies on a distance right to 2^-10.
+    const bool noisy = !ANY && TRI == kTriReference && variant == 0 && !(a.wide_size <= 1.0f);
+    if (a.wide && !noisy) {
         // refill 0 and the count known here: sweeps of 4 groups per wave, taking rays at 32
         // idle lanes. Against one wave per group and one persistent range (us): 1M shadow
         // rays 556 / 386, with sweeps 389; 1.8M rays in 250k triangles 960 / 846, 846, its

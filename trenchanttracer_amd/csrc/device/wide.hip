@@ -50,7 +50,9 @@ struct WideBuild {
     int2 *list;
     int32_t *last_of;       // [triangle id]: first unit of its record linked last, or -1
     int32_t ids;            // triangle ids below this have a ring; others stand alone
-    int32_t *state;         // [0] nodes listed, [1] records allocated, [2] set: the tree does not fit
+    // [0] nodes listed, [1] records allocated, [2] set: the tree does not fit, [3] bits of the
+    // largest |e1|^2 |e2|^2 of a triangle
+    int32_t *state;
     int32_t node_cap, rec_cap;
 };
 
@@ -126,12 +128,14 @@ __device__ int wave_scan(int v, int *total) {   // exclusive sum over the wave's
     return s - v;
 }
 
-__device__ void copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_t place, int32_t at, bool last) {
+__device__ float copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_t place, int32_t at, bool last) {
+    float size = 0.0f;
     const float4 *t = b.tris + (int64_t)~ref * 3;
     for (int i = 0; i < count; ++i) {
         const int32_t unit = b.step * (at + i);
         float4 *to = reinterpret_cast<float4 *>(b.wide) + unit;
         float4 e1 = t[3 * i + 1], e2 = t[3 * i + 2];
+        size = fmaxf(size, (e1.x * e1.x + e1.y * e1.y + e1.z * e1.z) * (e2.x * e2.x + e2.y * e2.y + e2.z * e2.z));
         const int32_t id = __float_as_int(t[3 * i].w);
         // the record before this one in the ring; the first closes it (k_wide_rings)
         int32_t link = id >= 0 && id < b.ids ? atomicExch(&b.last_of[id], unit) : unit;
@@ -142,6 +146,7 @@ __device__ void copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_
         to[1] = e1;
         to[2] = e2;
     }
+    return size;
 }
 
 // Closes the rings: the record linked first (it holds kRingEnd) points to the one linked
@@ -294,6 +299,7 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
     }
     uint32_t offsets = 0;
     int32_t off = 0;
+    float size = 0.0f;
     for (int k = 0; k < n; ++k) {
         if (c[k].count == 0) {
             b.list[node0 + k] = make_int2(rec0 + k, c[k].place);
@@ -302,10 +308,13 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
             continue;
         }
         offsets |= (uint32_t)(128 | b.step * off) << (8 * k);
-        copy_leaf(b, c[k].ref, c[k].count, c[k].place, rec0 + off, c[k].count2 == 0);
-        if (c[k].count2) copy_leaf(b, c[k].ref2, c[k].count2, c[k].place2, rec0 + off + c[k].count, true);
+        size = fmaxf(size, copy_leaf(b, c[k].ref, c[k].count, c[k].place, rec0 + off, c[k].count2 == 0));
+        if (c[k].count2)
+            size = fmaxf(size, copy_leaf(b, c[k].ref2, c[k].count2, c[k].place2, rec0 + off + c[k].count, true));
         off += c[k].count + c[k].count2;
     }
+    // (the value is only ever raised, so most threads find it high enough)
+    if (__float_as_int(size) > b.state[3]) atomicMax(&b.state[3], __float_as_int(size));
     if (no_leaf) {
         // no edges (never accepted), no triangle, its own ring, the end of its leaf
         const int32_t unit = b.step * (rec0 + off);
@@ -450,6 +459,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     }
     s->wide = mem;
     s->wide_step = step;
+    std::memcpy(&s->wide_size, &state[3], 4);
     s->wide_bound = (float)(bound * (1.0 + 4.0 / 255.0)) * 1.0001f;
     s->bytes += bytes;
     return TT_OK;
