@@ -586,8 +586,12 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                         hit_rec = (int)rec;
                         hit_place = fb(B.w);
                         cull = fb(t * 1.0009765625f);
-                    } else if (t > hit_t || fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)hit_rec)->w) != fb(A.w)) {
-                        next_t = fminf(next_t, t);   // (at hit_t itself: unless it is the same triangle again)
+                    } else if (hit_rec >= 0 &&
+                               (t > hit_t ||
+                                fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)hit_rec)->w) != fb(A.w))) {
+                        // (at hit_t itself: unless it is the same triangle again. Without a winner a
+                        // triangle at or past tmax is no hit, and next_t is tmax already.)
+                        next_t = fminf(next_t, t);
                     }
                 }
             }
