@@ -26,13 +26,13 @@ def _check(tt, oracle, scene, bvh, rays, what, cfgs=CFGS):
 
 
 def _soup_over_plane(tt):
-    """20000 small triangles in the unit cube over the plane z = 0, tessellated in
-    right triangles with legs of 0.5 (front faces up)."""
-    soup = tt.Mesh.soup(20000, seed=6).arrays()
-    x, y = np.meshgrid(np.arange(-4, 9) * 0.5, np.arange(-4, 9) * 0.5)
+    """20000 triangles in the unit cube (enough for the four-child tree) over the plane z = 0
+    from -0.5 to 1.5, tessellated in right triangles with legs of 0.25 (front faces up)."""
+    soup = tt.Mesh.soup(20000, seed=6, mu=float(np.log(0.03))).arrays()
+    x, y = np.meshgrid(np.arange(-2, 7) * 0.25, np.arange(-2, 7) * 0.25)
     v = np.stack([x.ravel(), y.ravel(), np.zeros(x.size)], 1)
-    a = (np.arange(12)[:, None] * 13 + np.arange(12)).ravel()
-    t = np.concatenate([np.stack([a, a + 1, a + 13], 1), np.stack([a + 14, a + 13, a + 1], 1)])
+    a = (np.arange(8)[:, None] * 9 + np.arange(8)).ravel()
+    t = np.concatenate([np.stack([a, a + 1, a + 9], 1), np.stack([a + 10, a + 9, a + 1], 1)])
     return tt.Mesh.from_arrays(np.concatenate([soup["verts"], v]).astype(np.float32),
                                np.concatenate([soup["tris"], t + len(soup["verts"])]).astype(np.int32))
 
@@ -46,8 +46,9 @@ def test_segments_ending_on_a_surface(tt, oracle, ctx):
     rng = np.random.default_rng(1)
     n = 4000
     down = np.zeros((n, 8), np.float32)
-    # outside the cube nothing lies before the plane; in it, sometimes
-    down[:, :2] = np.concatenate([rng.integers(-16, 0, (n // 2, 2)), rng.integers(0, 9, (n // 2, 2))]) / 8.0 + 0.0625
+    # beside the cube nothing lies before the plane; over it, mostly
+    down[:, :2] = rng.integers(-4, 12, (n, 2)) / 8.0 + 0.03125
+    down[:3 * n // 4, 0] = -np.abs(down[:3 * n // 4, 0] % 0.375) - 0.0625
     down[:, 2] = down[:, 7] = rng.choice([0.25, 0.5, 1.0, 2.0, 5.0], n)
     down[:, 6] = -1.0
     free = np.concatenate([tt.rays_incoherent(mesh, 20000, seed=3),
