@@ -263,15 +263,17 @@ tt_status tt_scene_set_geometries(tt_scene *s, const tt_geometry *g, int32_t n);
  * FP64 total weight (sum of luminance * sin(theta) over texels). */
 tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double *total);
 
-/* Traversal launch tuning. variant (scenes of short rays, which keep the two-child loop;
- * elsewhere both give the same walk and records): 0 = per-lane exact (single-lane order;
- * hit ids bit-identical to the host reference traversal), 1 = speculative while-while
- * (Aila-Laine postponed leaf + wave ballot). The four-child walk gives the host's records
- * too, but for triangles whose computed distance is rounding noise, more than 2^-10 below
- * their own box: of 5M rays aimed within 1e-8 to 1e-2 of the planes of triangles 5 to 20
- * units wide, 8 records differ (the speculative loop: 4; rays not aimed so: none of 400M).
- * Closest-hit calls of variant 0 therefore keep the two-child loop on scenes with a
- * triangle whose edges' lengths multiply to more than 1. lds_stack: LDS stack entries of 4 bytes per
+/* Traversal launch tuning. variant: 0 = exact (the records of the host reference traversal
+ * in single-lane order, bit for bit), 1 = fast: the records can differ where a computed
+ * distance is rounding noise, more than 2^-10 below the triangle's own box (of 5M rays aimed
+ * within 1e-8 to 1e-2 of the planes of triangles 5 to 20 units wide, 8 differ; rays not aimed
+ * so: none of 400M) and, on scenes of short rays (speculative while-while loop of Aila-Laine:
+ * postponed leaf + wave ballot), at near ties. Other scenes have a four-child tree. Exact
+ * rays walk it with boxes widened by what a computed hit can lie off its triangle, which the
+ * lengths of the edges, the direction and the distance bound; where triangles are large or
+ * far for that (several units, or scenes of tens of units in triangles of 0.1) closest-hit
+ * launches of variant 0 keep the two-child loop, and rays from further away than the tree is
+ * good for, or with longer directions, walk the two-child tree. lds_stack: LDS stack entries of 4 bytes per
  * lane (8, 16, 24 or 32; a closest-hit entry of the four-child walk is 8 bytes, and 3/4 of
  * the number of them are kept in LDS); block: threads per block (64..256, multiple of 64).
  * refill: 0 (default) = the library's choice: sweeps over one part of the range after
@@ -601,6 +603,10 @@ tt_status tt_debug_env_invert(tt_scene *s, const float *u, int64_t n, int32_t *o
  * read on the device (the path tracer's form); cap <= n, with the length from the
  * host. Synchronous. */
 tt_status tt_debug_ray_order(tt_scene *s, const tt_ray *rays, int64_t n, int64_t cap, int32_t *order);
+/* Which walk a scene's rays take: four_child = 1 if it has the four-child tree; reach = the
+ * largest |d| times distance from the origin to the far corner of the scene's box at which
+ * closest-hit rays of variant 0 walk it too (0: their launches take the two-child loop). */
+tt_status tt_debug_scene_walk(const tt_scene *s, int32_t *four_child, float *reach);
 
 #ifdef __cplusplus
 } /* extern "C" */

@@ -1,9 +1,12 @@
-"""The four-child closest-hit walk where a record depends on one comparison: segments that
-end exactly on a surface, against the oracle's single-lane walk."""
+"""The four-child closest-hit walk where a record depends on one comparison or on rounding:
+segments that end exactly on a surface, rays nearly in their triangles' planes, and the
+scenes of test_gpu_wide.py at scales at which exact rays take that walk; against the
+oracle's single-lane walk."""
 import sys
 
 import numpy as np
 import pytest
+import test_gpu_wide
 
 pytestmark = pytest.mark.gpu
 
@@ -43,6 +46,7 @@ def test_segments_ending_on_a_surface(tt, oracle, ctx):
     mesh = _soup_over_plane(tt)
     bvh = tt.BVH.build(mesh)
     scene = tt.DeviceScene(ctx, mesh, bvh)
+    assert scene.walk()[0] and scene.walk()[1] > 0.0
     rng = np.random.default_rng(1)
     n = 4000
     down = np.zeros((n, 8), np.float32)
@@ -63,4 +67,71 @@ def test_segments_ending_on_a_surface(tt, oracle, ctx):
         rays = free.copy()
         rays[:, 7] = end
         _check(tt, oracle, scene, bvh, rays, name)
+    scene.close()
+
+
+EXACT = tuple(c for c in CFGS if c[0] == 0)
+
+
+def _triangles(seed, tris, size, extent):
+    """Random triangles in a cube, |e1| |e2| up to size^2."""
+    rng = np.random.default_rng(seed)
+    v = rng.uniform(-extent, extent, (tris, 1, 3)) + rng.normal(0, 1, (tris, 3, 3)) * size
+    p = np.linalg.norm(v[:, 1] - v[:, 0], axis=1) * np.linalg.norm(v[:, 2] - v[:, 0], axis=1)
+    c = v.mean(1, keepdims=True)
+    return rng, (c + (v - c) * np.sqrt(np.minimum(1, 0.99 * size * size / p))[:, None, None]).astype(np.float32)
+
+
+def _grazing(rng, v, n, near, far):
+    """Rays at random points of the triangles v from near to far away, nearly in their
+    planes: det from the 1e-5 it is accepted from to ten times that."""
+    t = v[rng.integers(len(v), size=n)].astype(np.float64)
+    p = (t * rng.dirichlet((1, 1, 1), n)[:, :, None]).sum(1)
+    e1, e2 = t[:, 1] - t[:, 0], t[:, 2] - t[:, 0]
+    nn = np.cross(e1, e2)
+    nn /= np.linalg.norm(nn, axis=1, keepdims=True)
+    a = rng.uniform(0, 2 * np.pi, n)
+    u = e1 / np.linalg.norm(e1, axis=1, keepdims=True)
+    pr = np.linalg.norm(e1, axis=1) * np.linalg.norm(e2, axis=1)
+    off = 1e-5 / pr * 10 ** rng.uniform(0, 1.0, n)
+    d = u * np.cos(a)[:, None] + np.cross(nn, u) * np.sin(a)[:, None] - nn * off[:, None]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, :3] = p - d * (10 ** rng.uniform(np.log10(near), np.log10(far), n))[:, None]
+    rays[:, 4:7], rays[:, 7] = d, 1e20
+    return rays
+
+
+# the last column: whether exact rays from within the scene take the four-child walk there
+@pytest.mark.parametrize("seed,tris,size,extent,near,far,wide", [
+    (2, 2000, 1.0, 4, 30, 1000, False), (3, 20000, 1.0, 10, 10, 1000, False),
+    (4, 2000, 0.4, 0.5, 0.1, 10, False), (7, 20000, 0.1, 1, 0.1, 10, True), (8, 20000, 0.1, 1, 10, 1000, True),
+    (9, 200000, 0.05, 1, 0.1, 10, True), (10, 20000, 0.05, 0.3, 0.01, 3, True), (11, 3000, 0.2, 0.5, 0.03, 3, True)])
+def test_variant_0_is_exact_for_grazing_rays(tt, oracle, ctx, seed, tris, size, extent, near, far, wide):
+    _say(f"grazing rays: {tris} triangles of size {size} in {extent}, {near} to {far} away")
+    rng, v = _triangles(seed, tris, size, extent)
+    mesh = tt.Mesh.from_arrays(v.reshape(-1, 3), np.arange(3 * tris, dtype=np.int32).reshape(-1, 3))
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    assert scene.walk()[0] and (scene.walk()[1] > 0.0) == wide
+    rays = _grazing(rng, v, 1_000_000, near, far)
+    rays[::7, 4:7] *= 0.25   # lengths other than 1
+    rays[1::7, 4:7] *= 3.0
+    _check(tt, oracle, scene, bvh, rays, "grazing", EXACT)
+    scene.close()
+
+
+@pytest.mark.parametrize("kind,scale", [("layers", 2.0 ** -3), ("layers", 2.0 ** -5), ("hills", 2.0 ** -3),
+                                        ("hills", 2.0 ** -5), ("coincident", 2.0 ** -4), ("piles", 2.0 ** -5),
+                                        ("spread", 2.0 ** -4)])
+def test_exact_four_child_walk_matches_oracle(tt, oracle, ctx, kind, scale):
+    """test_gpu_wide.py's scenes and rays, small enough for exact rays to take the
+    four-child walk."""
+    _say(f"exact four-child walk: {kind} at {scale}")
+    a = test_gpu_wide._mesh(tt, kind).arrays()
+    mesh = tt.Mesh.from_arrays(a["verts"] * np.float32(scale), a["tris"])
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    assert scene.walk()[1] > 0.0
+    _check(tt, oracle, scene, bvh, test_gpu_wide._rays(mesh, 5), kind)
     scene.close()

@@ -710,6 +710,12 @@ class DeviceScene:
         check(lib.tt_debug_ray_order(self._h, C.c_void_p(d_rays.ptr), int(n), int(cap), _vp(out)))
         return out
 
+    def walk(self):
+        """(has the four-child tree, reach of exact closest hits on it) (tt_debug_scene_walk)."""
+        wide, reach = C.c_int32(), C.c_float()
+        check(lib.tt_debug_scene_walk(self._h, C.byref(wide), C.byref(reach)))
+        return bool(wide.value), reach.value
+
     def env_samples(self, n, seed=1):
         out = np.empty((int(n), 8), np.float32)
         check(lib.tt_debug_env_sample(self._h, int(n), int(seed), _vp(out)))

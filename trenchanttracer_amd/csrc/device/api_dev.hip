@@ -104,8 +104,14 @@ TraceArgs trace_args(const tt_scene *s) {
     a.num_nodes = (int32_t)s->num_nodes;
     a.wide = reinterpret_cast<const uint4 *>(s->wide);
     a.wide_step = s->wide_step;
-    a.wide_size = s->wide_size;
     a.wide_bound = s->wide_bound;
+    for (int q = 0; q < 3; ++q) {
+        a.wide_mid[q] = s->wide_mid[q];
+        a.wide_half[q] = s->wide_half[q];
+    }
+    a.wide_noise = s->wide_noise;
+    a.wide_grain = s->wide_grain;
+    a.wide_reach = s->wide_reach;
     a.roots = s->roots;
     return a;
 }
@@ -632,6 +638,13 @@ tt_status tt_debug_ray_order(tt_scene *s, const tt_ray *rays, int64_t n, int64_t
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     hipFree(ws);
     if (e != hipSuccess) return fail(TT_ERR_DEVICE, std::string("tt_debug_ray_order: ") + hipGetErrorString(e));
+    return TT_OK;
+}
+
+tt_status tt_debug_scene_walk(const tt_scene *s, int32_t *four_child, float *reach) {
+    if (!s || !four_child || !reach) return fail(TT_ERR_INVALID, "tt_debug_scene_walk: null argument");
+    *four_child = s->wide ? 1 : 0;
+    *reach = s->wide_reach;
     return TT_OK;
 }
 

@@ -54,6 +54,21 @@ __device__ __forceinline__ int32_t queue_slot(const Queue &q, int32_t r) {
     return i < q.counts[s * kSegStride] ? s * q.seg + i : -1;
 }
 
+// How far from its triangle a hit accepted by the reference's test can lie. With n = 2^-24 and
+// w = o - v0, the test computes pv = d x e2 and qv = w x e1 to 2.42 n of the product of the
+// factors' lengths (1.42 from the products, 1 from the differences), and from them det = e1 pv,
+// Nu = w pv, Nv = d qv and Nt = e2 qv, each sum of three products to 2 n of its factors' lengths
+// and its last rounding. Exactly, det w + Nt d = Nu e1 + Nv e2. An error e of pv enters that as
+// (e1 e) w - (w e) e1 = e x (w x e1), one of qv in the same way, so together 4.84 n |e1||e2||d||w|,
+// and the four sums 8 n of it. Hence, but for the unamplified roundings (of w, the last ones of
+// the sums, the divide: 9 n of the coordinates),
+//   |o + t d - (v0 + u e1 + v e2)| <= 12.9 n |e1||e2||d||w| / det,   det > 1e-5.
+// (The largest found over 20M accepted rays nearly in their triangles' planes, edges of 1e-3 to
+// 50, from 0.01 to 1000 away: 5.0 n.) The factor holds 1% for its own rounding.
+constexpr float kNoise = 12.9f * 0x1p-24f / 1e-5f * 1.01f;
+
+constexpr float kUnitLength = 1.02f;   // directions up to this length count as unit ones
+
 struct TraceArgs {
     const float4 *nodes;   // 4 float4 per node
     const float4 *tris;    // 3 float4 per triangle record
@@ -64,8 +79,11 @@ struct TraceArgs {
     int32_t num_nodes;
     const uint4 *wide;        // four-child tree and its triangle records (nullptr: walk the two-child one)
     int32_t wide_step;        // 16-byte units from one record of it to the next
-    float wide_size;          // largest |e1|^2 |e2|^2 of a triangle
     float wide_bound;         // largest coordinate of a plane
+    float wide_mid[3], wide_half[3];   // the scenes' box: centre and half extent (rounded up)
+    float wide_noise;         // kNoise times the unit of the nodes' size codes (wide.hip)
+    float wide_grain;         // length the sizes are taken against
+    float wide_reach;         // exact closest hit: largest |d| times distance across the scenes
     const int32_t *ray_root;  // if set: scene of each ray (its root is that record of the wide tree)
     const int32_t *roots;     // if set: the scenes' roots in the two-child tree
     const int32_t *n_dev;  // if set: ray count read on the device (capped at n), or with seg set ...

@@ -41,8 +41,9 @@ struct tt_scene {
     int64_t num_tris = 0;
     void *wide = nullptr;        // the four-child tree the traversal walks, with its triangle records (wide.hip)
     int32_t wide_step = 3;       // 16-byte units from one record of it to the next
-    float wide_size = 0.0f;      // largest |e1|^2 |e2|^2 of a triangle
     float wide_bound = 0.0f;
+    float wide_mid[3] = {}, wide_half[3] = {};
+    float wide_noise = 0.0f, wide_grain = 0.0f, wide_reach = 0.0f;   // see TraceArgs
     int32_t *roots = nullptr;    // several scenes in one tree: their two-child roots
     // shading data by original triangle id
     void *tri_normals = nullptr;  // float4 x 3 per triangle

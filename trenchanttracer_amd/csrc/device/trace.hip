@@ -27,14 +27,14 @@
 // (the first one visited wins there), or the ray is one the quantised arithmetic does not
 // cover (non-finite or overflowing terms, negative tmin, a full stack), the lane walks the
 // two-child tree. An any-hit ray applies the leaf test to every triangle it would accept.
-// (Boxes are culled against the best distance with 2^-10 to spare: a triangle whose
-// computed t lies further than that below its own box could still be skipped. That takes
-// |det| near the 1e-5 it is accepted from and edges whose product is large against it: of
-// 5M rays aimed within 1e-8 to 1e-2 of the planes of triangles 5 to 20 units wide, 8 got
-// another hit than the single-lane order's, which were at distances such as 4.0 for a
-// triangle 11.8 away; of 3M at triangles around one unit, none. A margin of 2^-6 finds no
-// more of them and costs 1.5 to 4%. So variant 0 keeps the two-child loop where triangles
-// are that large: launch_v. The speculative loop had such misses, 4 of those 5M.)
+// That rests on a culled box holding no triangle nearer than the best distance. In exact
+// arithmetic a hit lies in its triangle's box; a computed one can lie far off it, as |det|
+// goes down to 1e-5. For variant 0 (EXACT) boxes are widened by as much as it can (kNoise), so
+// that at any t the ray is inside every box down to one of the triangle's leaves and the
+// triangle is tested unless t is past the best distance. Variant 1 and path mode cull with
+// 2^-10 of the distance to spare instead: of 5M rays aimed within 1e-8 to 1e-2 of the planes
+// of triangles 5 to 20 units wide, 8 got another hit than the single-lane order's (the
+// speculative two-child loop: 4); of 9M at |e1||e2| up to 1 from up to 1000 units away, 3.
 //
 // Stack: the lowest S entries of each lane live in LDS ([entry][lane] so the lanes of a
 // wave hit distinct banks), deeper entries in per-lane scratch.
@@ -277,16 +277,26 @@ __device__ __forceinline__ bool in_leaf(const TraceArgs &a, int place, const Ray
 // `place`, while its best distance is t or more, through any of its leaves: the records of
 // one triangle form a ring (a spatial split puts a triangle in several leaves, and the one
 // it was found in here may be one whose own box the ray misses: 1-3% of the soup's rays).
-// Longer rings than the limit go to the full walk.
+// Longer rings than the limit go to the full walk, which a lane alone takes some 150 us for:
+// with a limit of 16, exact camera rays on soup of 250k triangles took 418 or 585 us by the
+// rings' order, which differs from one build of the tree to the next; with 64, 415.
 __device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, const RayTerms &r, float t) {
     if (in_leaf(a, place, r, t)) return true;
     int at = rec;
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 64; ++i) {
         at = fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[2].w) & 0x7FFFFFFF;
         if (at == rec) return false;
         if (in_leaf(a, fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[1].w), r, t)) return true;
     }
     return false;
+}
+
+// EXACT: what boxes are widened by for the sake of hits at t or nearer. Such a hit's |o - v0|
+// is at most t |d|, the triangle's longer edge and the hit's own displacement; the size codes
+// hold the last two for directions of about unit length (wide.hip), others are not narrowed.
+__device__ __forceinline__ float noise_to(const TraceArgs &a, float dx, float dy, float dz, float t) {
+    const float len = sqrtf(dx * dx + dy * dy + dz * dz);
+    return len <= kUnitLength ? a.wide_noise * len * (t * len + a.wide_grain) : INFINITY;
 }
 
 // The counts of the queue traced, uniform, and the slot of its r-th position (-1: none).
@@ -322,6 +332,10 @@ __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
     return full ? min(6, 32 - __clz((int)full)) : 0;
 }
 
+// EXACT widens boxes as kNoise asks (9 instructions a node, 73 VGPRs as held to 6 waves per
+// SIMD, 82 without): soup of 250k triangles, 1.2M rays, 634 us as variant 1, 678 exact, of 20k
+// 448 and 506; with nothing to widen, 634 and 448.
+//
 // Four-child walk. What bounds it: VALU issue first, vector memory lane loads second. On
 // the 1M-triangle soup (8.3M rays in Morton order) the two-child while-while loop kept VALU
 // issue 90% and the address path 82% busy, with 32% of the lanes active: 1.85e9 VALU
@@ -329,8 +343,9 @@ __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
 // instead of 8, and taking node visits and triangle tests by the vote below (59% of the
 // lanes active), takes 1.43e9, 0.90e9 and 3.0 ms; each alone gains little, as the other
 // limit holds (four children in the while-while loop: 6.6 ms, slower).
-template <bool ANY, int S, int TRI>
-__global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
+template <bool ANY, int S, int TRI, bool EXACT>
+__global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) {
+    static_assert(!EXACT || (!ANY && TRI == kTriReference), "kNoise is the reference test's");
     using E = typename std::conditional<ANY, int, uint64_t>::type;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int tid = threadIdx.x;
@@ -392,6 +407,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
     float idirx = 0.0f, idiry = 0.0f, idirz = 0.0f;
     float nearx = 0.0f, neary = 0.0f, nearz = 0.0f;   // -(o idir) less the rounding allowance
     float farx = 0.0f, fary = 0.0f, farz = 0.0f;      // -(o idir) plus it
+    float noise = 0.0f;        // EXACT: what a node's boxes are widened by, over its size code squared
     int node = kSentinel;      // inner node to visit; sign set: a leaf waiting for room; kSentinel: none
     int leaf = 0, leaf2 = 0;   // sign set: next record of the leaf being tested, first of the one after it
     float hit_t = 0.0f;
@@ -451,9 +467,13 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                 // to 2^-53): the two-child test's terms are off by at most
                 // 2.01 (B + |o|) |idir| 2^-24 and this one's by 4.1 of the same, B the largest
                 // coordinate of a plane; 8 covers the two
-                const float sx = (fabsf(ox) + a.wide_bound) * fabsf(idirx) * 0x1p-21f;
-                const float sy = (fabsf(oy) + a.wide_bound) * fabsf(idiry) * 0x1p-21f;
-                const float sz = (fabsf(oz) + a.wide_bound) * fabsf(idirz) * 0x1p-21f;
+                // (EXACT: 32 instead, for what kNoise leaves out: besides this slab test's 4.1, 9 for
+                // the test's unamplified roundings, 2 for the edges', 9 for a spatial split's clipped
+                // boxes)
+                constexpr float kSlack = EXACT ? 0x1p-19f : 0x1p-21f;
+                const float sx = (fabsf(ox) + a.wide_bound) * fabsf(idirx) * kSlack;
+                const float sy = (fabsf(oy) + a.wide_bound) * fabsf(idiry) * kSlack;
+                const float sz = (fabsf(oz) + a.wide_bound) * fabsf(idirz) * kSlack;
                 nearx = -(ox * idirx) - sx;
                 neary = -(oy * idiry) - sy;
                 nearz = -(oz * idirz) - sz;
@@ -462,8 +482,19 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                 farz = sz - oz * idirz;
                 // rays the wide walk covers: all terms finite (NaN compares false), the
                 // allowance positive, distances that compare as integers
-                const bool fits = sx > 0.0f && sy > 0.0f && sz > 0.0f && sx < 1e30f && sy < 1e30f &&
-                                  sz < 1e30f && fb(tmin) >= 0 && tmin < 1e30f && fb(tmax) >= 0 && tmax <= INFINITY;
+                bool fits = sx > 0.0f && sy > 0.0f && sz > 0.0f && sx < 1e30f && sy < 1e30f &&
+                            sz < 1e30f && fb(tmin) >= 0 && tmin < 1e30f && fb(tmax) >= 0 && tmax <= INFINITY;
+                if constexpr (EXACT) {
+                    const float ax = fabsf(ox - a.wide_mid[0]) + a.wide_half[0];
+                    const float ay = fabsf(oy - a.wide_mid[1]) + a.wide_half[1];
+                    const float az = fabsf(oz - a.wide_mid[2]) + a.wide_half[2];
+                    const float dd = dx * dx + dy * dy + dz * dz;
+                    const float across = sqrtf(dd) * sqrtf(ax * ax + ay * ay + az * az);
+                    noise = min(a.wide_noise * across, noise_to(a, dx, dy, dz, tmax));
+                    const float most = noise * (255.0f * 255.0f);
+                    fits = fits && across <= a.wide_reach && dd > 1e-30f && most * fabsf(idirx) < 1e30f &&
+                           most * fabsf(idiry) < 1e30f && most * fabsf(idirz) < 1e30f;
+                }
                 st.clear();
                 redo = !fits;
                 leaf = leaf2 = 0;
@@ -514,9 +545,18 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                     const float ky = ldexpf(idiry, __builtin_amdgcn_sbfe((int)q1.y, 8, 8));
                     const float kz = ldexpf(idirz, __builtin_amdgcn_sbfe((int)q1.y, 16, 8));
                     const float bx = bf((int)q0.x), by = bf((int)q0.y), bz = bf((int)q0.z);
-                    const float nx = __builtin_fmaf(bx, idirx, nearx), fx = __builtin_fmaf(bx, idirx, farx);
-                    const float ny = __builtin_fmaf(by, idiry, neary), fy = __builtin_fmaf(by, idiry, fary);
-                    const float nz = __builtin_fmaf(bz, idirz, nearz), fz = __builtin_fmaf(bz, idirz, farz);
+                    float nx = __builtin_fmaf(bx, idirx, nearx), fx = __builtin_fmaf(bx, idirx, farx);
+                    float ny = __builtin_fmaf(by, idiry, neary), fy = __builtin_fmaf(by, idiry, fary);
+                    float nz = __builtin_fmaf(bz, idirz, nearz), fz = __builtin_fmaf(bz, idirz, farz);
+                    if constexpr (EXACT) {
+                        const float code = (float)(q1.y >> 24), pad = noise * code * code;
+                        nx = __builtin_fmaf(-pad, fabsf(idirx), nx);
+                        fx = __builtin_fmaf(pad, fabsf(idirx), fx);
+                        ny = __builtin_fmaf(-pad, fabsf(idiry), ny);
+                        fy = __builtin_fmaf(pad, fabsf(idiry), fy);
+                        nz = __builtin_fmaf(-pad, fabsf(idirz), nz);
+                        fz = __builtin_fmaf(pad, fabsf(idirz), fz);
+                    }
                     const bool px = idirx >= 0.0f, py = idiry >= 0.0f, pz = idirz >= 0.0f;
                     const uint32_t nwx = px ? q1.z : q1.w, fwx = px ? q1.w : q1.z;
                     const uint32_t nwy = py ? q2.x : q2.y, fwy = py ? q2.y : q2.x;
@@ -586,6 +626,7 @@ __global__ __launch_bounds__(256) void k_trace_wide(TraceArgs a) {
                         hit_rec = (int)rec;
                         hit_place = fb(B.w);
                         cull = fb(t * 1.0009765625f);
+                        if constexpr (EXACT) noise = min(noise, noise_to(a, dx, dy, dz, bf(cull)));
                     } else if (hit_rec >= 0 &&
                                (t > hit_t ||
                                 fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)hit_rec)->w) != fb(A.w))) {
@@ -880,15 +921,15 @@ hipError_t launch_k(K kernel, TraceArgs a, bool persistent, int block, size_t ld
     return hipGetLastError();
 }
 
-template <bool ANY, int TRI>
+template <bool ANY, int TRI, bool EXACT>
 hipError_t launch_wide(const TraceArgs &a, bool persistent, int S, int block, int num_cus, hipStream_t s) {
     // S entries for any-hit launches (4 bytes each), 3/4 S for closest-hit ones (8 bytes)
     const size_t lds = (ANY ? (size_t)S * 4 : (size_t)S * 6) * block;
     switch (S) {
-        case 8: return launch_k(k_trace_wide<ANY, ANY ? 8 : 6, TRI>, a, persistent, block, lds, num_cus, s);
-        case 16: return launch_k(k_trace_wide<ANY, ANY ? 16 : 12, TRI>, a, persistent, block, lds, num_cus, s);
-        case 24: return launch_k(k_trace_wide<ANY, ANY ? 24 : 18, TRI>, a, persistent, block, lds, num_cus, s);
-        case 32: return launch_k(k_trace_wide<ANY, ANY ? 32 : 24, TRI>, a, persistent, block, lds, num_cus, s);
+        case 8: return launch_k(k_trace_wide<ANY, ANY ? 8 : 6, TRI, EXACT>, a, persistent, block, lds, num_cus, s);
+        case 16: return launch_k(k_trace_wide<ANY, ANY ? 16 : 12, TRI, EXACT>, a, persistent, block, lds, num_cus, s);
+        case 24: return launch_k(k_trace_wide<ANY, ANY ? 24 : 18, TRI, EXACT>, a, persistent, block, lds, num_cus, s);
+        case 32: return launch_k(k_trace_wide<ANY, ANY ? 32 : 24, TRI, EXACT>, a, persistent, block, lds, num_cus, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -909,11 +950,10 @@ hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int n
 // the two-child loop of the asked variant elsewhere.
 template <bool ANY, int TRI>
 hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int block, int num_cus, hipStream_t s) {
-    // The exact loop is asked for and triangles are so large that the distance of one accepted
-    // at |det| > 1e-5 can be rounding noise (about 1e-2 |e1| |e2| of it): the two-child walk,
-    // as the culling of the four-child one relies on a distance right to 2^-10.
-    const bool noisy = !ANY && TRI == kTriReference && variant == 0 && !(a.wide_size <= 1.0f);
-    if (a.wide && !noisy) {
+    // exact closest hits: on scenes where kNoise's widened boxes pay (wide_reach: build_wide)
+    constexpr bool kBounded = !ANY && TRI == kTriReference;
+    const bool exact = kBounded && variant == 0;
+    if (a.wide && !(exact && !(a.wide_reach > 0.0f))) {
         // refill 0 and the count known here: sweeps of 4 groups per wave, taking rays at 32
         // idle lanes. Against one wave per group and one persistent range (us): 1M shadow
         // rays 556 / 386, with sweeps 389; 1.8M rays in 250k triangles 960 / 846, 846, its
@@ -926,7 +966,8 @@ hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int
             b.sweep = 4;
             b.refill = 32;
         }
-        return launch_wide<ANY, TRI>(b, persistent || b.sweep, S, block, num_cus, s);
+        if (exact) return launch_wide<ANY, TRI, kBounded>(b, persistent || b.sweep, S, block, num_cus, s);
+        return launch_wide<ANY, TRI, false>(b, persistent || b.sweep, S, block, num_cus, s);
     }
     if (variant == 0) return launch_s<0, ANY, TRI>(a, persistent, S, block, num_cus, s);
     if (variant == 1) return launch_s<1, ANY, TRI>(a, persistent, S, block, num_cus, s);
