@@ -273,7 +273,8 @@ tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double 
  * lengths of the edges, the direction and the distance bound; where triangles are large or
  * far for that (several units, or scenes of tens of units in triangles of 0.1) closest-hit
  * launches of variant 0 keep the two-child loop, and rays from further away than the tree is
- * good for, or with longer directions, walk the two-child tree. lds_stack: LDS stack entries of 4 bytes per
+ * good for, or with longer directions, walk the two-child tree. So do path mode's with
+ * variant 0, whose two-sided test bounds nothing. lds_stack: LDS stack entries of 4 bytes per
  * lane (8, 16, 24 or 32; a closest-hit entry of the four-child walk is 8 bytes, and 3/4 of
  * the number of them are kept in LDS); block: threads per block (64..256, multiple of 64).
  * refill: 0 (default) = the library's choice: sweeps over one part of the range after
@@ -396,7 +397,8 @@ typedef struct tt_render_params {
                                  scenes), 232 B more with a guide; guided renders that train the network: about 8M) */
     int32_t lds_stack;        /* traversal LDS stack entries per lane (0 = 16) */
     int32_t block;            /* traversal block size (0 = 64) */
-    int32_t variant;          /* path-mode traversal loop: -1 speculative (default), 0 exact, 1 speculative */
+    int32_t variant;          /* path mode's closest-hit traversal (see tt_trace_cfg): -1 = 1 (default), 0 exact
+                                 (the two-child loop), 1 fast */
     int32_t refill_camera;    /* traversal refill (see tt_trace_cfg) for the camera rays (0 = one wave per group) */
     int32_t refill;           /* ... for every later extension and shadow launch (0 = persistent, 40) */
     int32_t tile;             /* path slots walk tile x tile pixel blocks (0 = 8; 1 = pixel rows; 2..32);

@@ -135,3 +135,36 @@ def test_exact_four_child_walk_matches_oracle(tt, oracle, ctx, kind, scale):
     assert scene.walk()[1] > 0.0
     _check(tt, oracle, scene, bvh, test_gpu_wide._rays(mesh, 5), kind)
     scene.close()
+
+
+@pytest.mark.parametrize("seed,tris,size,spread,fov", [(4, 30, 2.0, 0.0, 1e-5), (6, 100, 1.0, 0.0, 1e-6),
+                                                       (8, 400, 0.6, 3e-6, 1e-5)])
+def test_path_mode_variant_0_is_exact_for_grazing_rays(tt, ctx, seed, tris, size, spread, fov):
+    """A camera almost in the plane of large triangles, whose two-sided test accepts any
+    determinant but 0: the image of the same scene with a triangle far away, which leaves
+    the rest of the tree (without spatial splits) as it is and makes the scene one whose
+    rays take the two-child loop."""
+    _say(f"grazing camera rays: {tris} triangles of size {size}")
+    rng = np.random.default_rng(seed)
+    centre = np.stack([rng.uniform(0, 20, tris), rng.uniform(-10, 10, tris), rng.normal(0, spread, tris)], 1)
+    flat = centre[:, None] + rng.normal(0, 1, (tris, 3, 3)) * np.array([size, size, 1e-6])
+    centre = np.stack([rng.uniform(0, 20, 3000), rng.uniform(-10, 10, 3000), rng.uniform(-10, 10, 3000)], 1)
+    v = np.concatenate([flat, centre[:, None] + rng.normal(0, 0.3, (3000, 3, 3))]).reshape(-1, 3)
+    rot, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+    v = v @ rot.T
+    mats = [tt.material(tt.MAT_DIFFUSE, (0.5, 0.5, 0.5), emission=(k + 1.0, float(k * k), 1.0)) for k in range(61)]
+    cam = tt.camera(tuple(rot @ [-3.0, 0.3, 0.0]), tuple(rot @ [1.0, 0.013, 0.0]), up=tuple(rot @ [0.0, 0.0, 1.0]),
+                    fov=(60.0, fov), width=2048, height=1024)
+    prm = tt.render_params(spp=2, max_depth=1, seed=seed, mode=tt.RENDER_PATH, variant=0)
+    images = []
+    for away in (False, True):
+        w = np.concatenate([v, [[-5e3, -5e3, -5e3], [-5001, -5e3, -5e3], [-5e3, -5001, -5e3]]]) if away else v
+        t = np.arange(len(w), dtype=np.int32).reshape(-1, 3)
+        mesh = tt.Mesh.from_arrays(w.astype(np.float32), t, tri_mats=(np.arange(len(t)) % 61).astype(np.int32))
+        scene = tt.DeviceScene(ctx, mesh, tt.BVH.build(mesh, split_alpha=1e30), mats)
+        assert scene.walk()[0] != away
+        images.append(scene.render(cam, prm)[0])
+        scene.close()
+    assert (images[0] > 0).any(2).mean() > 0.2
+    bad = (images[0] != images[1]).any(2).sum()
+    assert bad == 0, f"{bad} pixels differ"

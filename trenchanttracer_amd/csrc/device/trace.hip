@@ -29,10 +29,11 @@
 // two-child tree. An any-hit ray applies the leaf test to every triangle it would accept.
 // That rests on a culled box holding no triangle nearer than the best distance. In exact
 // arithmetic a hit lies in its triangle's box; a computed one can lie far off it, as |det|
-// goes down to 1e-5. For variant 0 (EXACT) boxes are widened by as much as it can (kNoise), so
+// goes down to 1e-5. For variant 0 with the reference's test (EXACT) boxes are widened by as much as it can (kNoise), so
 // that at any t the ray is inside every box down to one of the triangle's leaves and the
-// triangle is tested unless t is past the best distance. Variant 1 and path mode cull with
-// 2^-10 of the distance to spare instead: of 5M rays aimed within 1e-8 to 1e-2 of the planes
+// triangle is tested unless t is past the best distance (with the two-sided test, which
+// accepts any det but 0, variant 0 takes the two-child loop). Variant 1 culls with 2^-10 of
+// the distance to spare instead: of 5M rays aimed within 1e-8 to 1e-2 of the planes
 // of triangles 5 to 20 units wide, 8 got another hit than the single-lane order's (the
 // speculative two-child loop: 4); of 9M at |e1||e2| up to 1 from up to 1000 units away, 3.
 //
@@ -950,10 +951,11 @@ hipError_t launch_s(const TraceArgs &a, bool persistent, int S, int block, int n
 // the two-child loop of the asked variant elsewhere.
 template <bool ANY, int TRI>
 hipError_t launch_v(const TraceArgs &a, bool persistent, int variant, int S, int block, int num_cus, hipStream_t s) {
-    // exact closest hits: on scenes where kNoise's widened boxes pay (wide_reach: build_wide)
+    // exact closest hits: by the reference's test, on scenes where kNoise's widened boxes pay
+    // (wide_reach: build_wide); the two-sided test accepts any det but 0, which bounds nothing
     constexpr bool kBounded = !ANY && TRI == kTriReference;
-    const bool exact = kBounded && variant == 0;
-    if (a.wide && !(exact && !(a.wide_reach > 0.0f))) {
+    const bool exact = !ANY && variant == 0;
+    if (a.wide && !(exact && !(kBounded && a.wide_reach > 0.0f))) {
         // refill 0 and the count known here: sweeps of 4 groups per wave, taking rays at 32
         // idle lanes. Against one wave per group and one persistent range (us): 1M shadow
         // rays 556 / 386, with sweeps 389; 1.8M rays in 250k triangles 960 / 846, 846, its
