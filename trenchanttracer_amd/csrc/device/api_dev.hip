@@ -603,13 +603,18 @@ static tt_status trace_impl(tt_scene *s, const tt_ray *rays, int64_t n, tt_hit *
         // the workspace is the context's: a call on another stream waits for the last
         // launch that read it
         if (ctx->reorder_pending) TT_HIP(hipStreamWaitEvent(hs, ctx->reorder_done, 0), "hipStreamWaitEvent");
-        TT_HIP(reorder_rays(rays, n, s->bmin, s->bmax, ctx->reorder_ws, sort_bytes, hs, &a.order), "trace: reorder");
+        const hipError_t sorted = reorder_rays(rays, n, s->bmin, s->bmax, ctx->reorder_ws, sort_bytes, hs, &a.order);
+        const hipError_t traced = sorted != hipSuccess ? hipSuccess : launch_trace(a, c.variant, any, c.lds_stack, c.block, c.xcd_order,
+                                                                                  c.refill, ctx->num_cus, hs);
+        // also after an error: what was launched until then uses the workspace
+        const hipError_t recorded = hipEventRecord(ctx->reorder_done, hs);
+        ctx->reorder_pending = ctx->reorder_pending || recorded == hipSuccess;
+        TT_HIP(sorted, "trace: reorder");
+        TT_HIP(traced, "trace launch");
+        TT_HIP(recorded, "hipEventRecord");
+        return TT_OK;
     }
     TT_HIP(launch_trace(a, c.variant, any, c.lds_stack, c.block, c.xcd_order, c.refill, s->ctx->num_cus, hs), "trace launch");
-    if (c.reorder && !noalloc) {
-        TT_HIP(hipEventRecord(s->ctx->reorder_done, hs), "hipEventRecord");
-        s->ctx->reorder_pending = true;
-    }
     return TT_OK;
 }
 

@@ -1013,12 +1013,14 @@ hipError_t launch_trace(const TraceArgs &a, int variant, bool any, int lds_stack
     // / 337. Guided render 12.75 / 12.58 / 12.58 / 12.69 / 13.29 ms, room of 20 triangles 2089
     // / 2091 / 2096 / 2106 / 2143 us.
     for (b.spread = 0; 8LL * std::max(1, num_cus) >> (b.spread + 1);) ++b.spread;
-    // ray indices are 32-bit in the kernel: more rays go in several launches (a device-side
-    // count or an order comes with fewer)
-    constexpr int64_t kPart = (int64_t)1 << 30;
-    if (a.n > kPart && (a.n_dev || a.order)) return hipErrorInvalidValue;
-    for (int64_t at = 0; at < a.n; at += kPart) {
-        b.n = std::min(kPart, a.n - at);
+    // ray indices are 32-bit in the kernel: more rays go in several launches, but one with a
+    // device-side count or an order, which have fewer
+    constexpr int64_t kMost = ((int64_t)1 << 31) - 1;
+    const bool whole = a.n_dev || a.order;
+    if (whole && a.n > kMost) return hipErrorInvalidValue;
+    const int64_t part = whole ? a.n : (int64_t)1 << 30;
+    for (int64_t at = 0; at < a.n; at += part) {
+        b.n = std::min(part, a.n - at);
         b.rays = a.rays + at;
         if (a.hits) b.hits = a.hits + at;
         if (a.flags) b.flags = a.flags + at;
