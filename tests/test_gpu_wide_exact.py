@@ -168,3 +168,25 @@ def test_path_mode_variant_0_is_exact_for_grazing_rays(tt, ctx, seed, tris, size
     assert (images[0] > 0).any(2).mean() > 0.2
     bad = (images[0] != images[1]).any(2).sum()
     assert bad == 0, f"{bad} pixels differ"
+
+
+@pytest.mark.parametrize("kind,scale", [("layers", 2.0 ** -5), ("hills", 1.0), ("coincident", 2.0 ** -5)])
+def test_very_long_directions(tt, oracle, ctx, kind, scale):
+    """Directions up to 2^127 long, whose slab terms are denormal."""
+    a = test_gpu_wide._mesh(tt, kind).arrays()
+    mesh = tt.Mesh.from_arrays(a["verts"] * np.float32(scale), a["tris"])
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    base = test_gpu_wide._rays(mesh, 5)
+    longest = np.abs(base[:, 4:7]).max(1)
+    base = base[np.isfinite(base).all(1) & (longest > 0) & (base[:, 3] >= 0)]
+    longest = np.abs(base[:, 4:7]).max(1)
+    for k in (60, 79, 100, 118, 124, 127):
+        _say(f"very long directions: {kind} at {scale}, 2^{k}")
+        rays = base.copy()
+        rays[:, 4:7] = rays[:, 4:7] / longest[:, None] * np.float32(2.0 ** k)
+        rays[:, 3], rays[:, 7] = 0.0, 1e20
+        _check(tt, oracle, scene, bvh, rays, f"2^{k}")
+        want, _ = oracle.CompactBVH(bvh.export_compact()).trace(rays, any_hit=True, nthreads=8)
+        assert np.array_equal(scene.occluded(rays), (oracle.hit_ids(want) >= 0).astype(np.int32))
+    scene.close()

@@ -226,8 +226,8 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // LD: columns written and row stride of raw, kGuideNOutPad16 or the kGuideNOut real ones
-// (compiled in, so that the training forward and the renderer test no column: 49.4 us for
-// 262144 rows, 49.9 with a run-time stride)
+// (compiled in, so that the training forward and the renderer test no column: 49.3 us for
+// 262144 rows, 49.6 with a run-time stride)
 template <int LD>
 __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(InferArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];

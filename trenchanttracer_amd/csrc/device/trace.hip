@@ -481,9 +481,11 @@ __global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) 
                 farx = sx - ox * idirx;
                 fary = sy - oy * idiry;
                 farz = sz - oz * idirz;
-                // rays the wide walk covers: all terms finite (NaN compares false), the
-                // allowance positive, distances that compare as integers
-                bool fits = sx > 0.0f && sy > 0.0f && sz > 0.0f && sx < 1e30f && sy < 1e30f &&
+                // rays the wide walk covers: all terms finite (NaN compares false), the allowance
+                // far above what denormal terms lose (directions past about 2^79 of the scene's
+                // size do not), distances that compare as integers
+                constexpr float kLeast = 0x1p-100f;
+                bool fits = sx > kLeast && sy > kLeast && sz > kLeast && sx < 1e30f && sy < 1e30f &&
                             sz < 1e30f && fb(tmin) >= 0 && tmin < 1e30f && fb(tmax) >= 0 && tmax <= INFINITY;
                 if constexpr (EXACT) {
                     const float ax = fabsf(ox - a.wide_mid[0]) + a.wide_half[0];
