@@ -190,3 +190,22 @@ def test_very_long_directions(tt, oracle, ctx, kind, scale):
         want, _ = oracle.CompactBVH(bvh.export_compact()).trace(rays, any_hit=True, nthreads=8)
         assert np.array_equal(scene.occluded(rays), (oracle.hit_ids(want) >= 0).astype(np.int32))
     scene.close()
+
+
+@pytest.mark.parametrize("offset,wide", [(100.0, True), (1000.0, True), (30000.0, False)])
+def test_scenes_far_from_the_origin(tt, oracle, ctx, offset, wide):
+    """Coordinates large against the scene, whose rounding widens the four-child walk's
+    boxes: the records of the single-lane order, and no such walk where that costs more
+    than it gives."""
+    _say(f"scene at {offset}")
+    a = tt.Mesh.soup(20000, seed=6, mu=float(np.log(0.03))).arrays()
+    near = tt.Mesh.from_arrays(a["verts"], a["tris"])
+    mesh = tt.Mesh.from_arrays(a["verts"] + np.float32(offset), a["tris"])
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    assert scene.walk()[0] == wide
+    rays = np.concatenate([tt.rays_incoherent(near, 40000, seed=3),
+                           tt.rays_primary(200, 200, 1, (0.5, 0.5, -1.0), (0.5, 0.5, 0.0), seed=3)])
+    rays[:, :3] += np.float32(offset)
+    _check(tt, oracle, scene, bvh, rays, "far from the origin", EXACT)
+    scene.close()

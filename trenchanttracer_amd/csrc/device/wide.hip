@@ -58,8 +58,8 @@ struct WideState {
     float most;               // the scenes' largest size (k_wide_sizes)
     // Boxes entered per line through the scenes' box (sums of the boxes' areas over its own),
     // 32 fractional bits (whole numbers: the same sum in any order): [0] the boxes as they are,
-    // [1 + k] widened for reach_of(k)
-    unsigned long long cost[1 + kReaches];
+    // [1] widened by the walk's rounding allowance, [2 + k] for exact hits up to reach_of(k)
+    unsigned long long cost[2 + kReaches];
 };
 
 struct WideBuild {
@@ -79,6 +79,7 @@ struct WideBuild {
     WideState *state;
     int32_t node_cap, rec_cap;
     float diagonal, area;     // of the scenes' box: length, half its surface
+    float slack;              // what the rounding allowance adds to a box's extents
     float per_grain;
 };
 
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(256) void k_wide_sizes(WideBuild b, int32_t count) 
     const int32_t i = blockIdx.x * 256 + threadIdx.x;
     float most = 0.0f;
     for (int32_t k = 0; k < b.nroots; ++k) most = fmaxf(most, __int_as_float(max(b.size[k], 0)));
-    unsigned long long cost[1 + kReaches] = {};
+    unsigned long long cost[2 + kReaches] = {};
     if (i < count) {
         if (i == 0) b.state->most = most;
         uint4 *w = b.wide + b.step * (i < b.nroots ? i : b.list[i].x);
@@ -386,15 +387,16 @@ __global__ __launch_bounds__(256) void k_wide_sizes(WideBuild b, int32_t count) 
                                  (int)(int8_t)(q.y >> 8 * c & 255));
             if (size[0] < 0.0f) continue;   // an empty slot
 #pragma unroll
-            for (int f = 0; f <= kReaches; ++f) {
-                const float pad = f ? unit * reach_of(f - 1) : 0.0f;
+            for (int f = 0; f < 2 + kReaches; ++f) {
+                // (exact hits' allowance is four times that of others: kSlack)
+                const float pad = f == 0 ? 0.0f : f == 1 ? b.slack : 4.0f * b.slack + unit * reach_of(f - 2);
                 const float x = size[0] + pad, y = size[1] + pad, z = size[2] + pad;
                 cost[f] += (unsigned long long)(fminf((x * y + y * z + z * x) / b.area, 1.0f) * 0x1p32f);
             }
         }
     }
 #pragma unroll
-    for (int f = 0; f <= kReaches; ++f) {
+    for (int f = 0; f < 2 + kReaches; ++f) {
         for (int o = 32; o > 0; o >>= 1) cost[f] += __shfl_down(cost[f], o);
         if (__lane_id() == 0 && cost[f]) atomicAdd(&b.state->cost[f], cost[f]);
     }
@@ -511,6 +513,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     }
     b.diagonal = (float)std::sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
     b.per_grain = 1.0f / (b.diagonal * kGrain);
+    b.slack = (float)bound * 0x1p-19f;   // two sides of 2^-21 (|o| + B), origins as far out as the scene
     b.area = (float)(x[0] * x[1] + x[1] * x[2] + x[2] * x[0]);
     b.node_cap = (int32_t)s->num_nodes;
     b.rec_cap = (int32_t)recs;
@@ -544,6 +547,14 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
         hipFree(mem);
         return err == hipSuccess ? TT_OK : fail(TT_ERR_DEVICE, std::string("scene tree: ") + hipGetErrorString(err));
     }
+    // Far from the coordinates' origin the rounding allowance widens the boxes, which the two-child
+    // walk has none of. Measured (400k rays, us, two-child loop / four-child walk): the unit cube of
+    // 50k triangles at 0 365 / 302, offset by 1000 359 / 336, by 10000 366 / 567, by 100000 433 / 7679.
+    const auto grown = [&](int k) { return (double)state.cost[k] / (double)state.cost[0]; };
+    if (!(grown(1) <= 1.3)) {
+        hipFree(mem);
+        return TT_OK;
+    }
     // Exact closest hits take the four-child walk where widening its boxes for rays from within
     // the scene adds less than 0.3 of them, and there for rays from as far away, or with
     // as long directions, as at most double them; the lanes of others walk the two-child tree.
@@ -552,12 +563,11 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     // 1015 / 958, 4 times 2.4 1015 / 1723; soup of 2000 1.22 466 / 376, 1.5 times 1.55 466 / 458;
     // 180k triangles of terrain 1.08 269 / 218, 1.24 269 / 259, 1.36 269 / 284; soup of 100k and a
     // floor quad 1.11 910 / 701, a larger one 1.47 910 / 1238. All rays too far: 1015 / 1637, 466 / 516.
-    const auto costs = [&](int k) { return (double)state.cost[1 + k] / (double)state.cost[0]; };
     s->wide_grain = b.diagonal * kGrain;
     s->wide_noise = kNoise * state.most / (255.0f * 255.0f);
     s->wide_reach = 0.0f;
-    if (state.most <= kMaxSize && costs(0) <= 1.3)
-        for (int k = 0; k < kReaches && costs(k) <= 2.0; ++k) s->wide_reach = b.diagonal * reach_of(k);
+    if (state.most <= kMaxSize && grown(2) <= 1.3)
+        for (int k = 0; k < kReaches && grown(2 + k) <= 2.0; ++k) s->wide_reach = b.diagonal * reach_of(k);
     s->wide = mem;
     s->wide_step = step;
     s->wide_bound = (float)(bound * (1.0 + 4.0 / 255.0)) * 1.0001f;
