@@ -265,7 +265,8 @@ tt_status tt_env_export_cdf(const tt_scene *s, float *marg, float *cond, double 
 
 /* Traversal launch tuning. variant: 0 = exact (the records of the host reference traversal
  * in single-lane order, bit for bit), 1 = fast: the records can differ where a computed
- * distance is rounding noise, more than 2^-10 below the triangle's own box (of 5M rays aimed
+ * distance is rounding noise, more than 2^-10 below the triangle's own box, or, from further
+ * than 4 scene sizes away, 2^-8 of the scene's size, at least 2^-16 (of 5M rays aimed
  * within 1e-8 to 1e-2 of the planes of triangles 5 to 20 units wide, 8 differ; rays not aimed
  * so: none of 400M) and, on scenes of short rays (speculative while-while loop of Aila-Laine:
  * postponed leaf + wave ballot), at near ties. Other scenes have a four-child tree. Exact

@@ -209,3 +209,29 @@ def test_scenes_far_from_the_origin(tt, oracle, ctx, offset, wide):
     rays[:, :3] += np.float32(offset)
     _check(tt, oracle, scene, bvh, rays, "far from the origin", EXACT)
     scene.close()
+
+
+def test_rays_from_far_away(tt, oracle, ctx):
+    """Origins 1 to 10^7 scene sizes away, around the distances at which the culling margin
+    and the walk change: variant 0's records and any hit's flags; variant 1's distances to
+    rounding."""
+    mesh = tt.Mesh.soup(20000, seed=6, mu=float(np.log(0.03)))
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    rng = np.random.default_rng(1)
+    n = 20000
+    at, d = rng.random((n, 3)), rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    cb = oracle.CompactBVH(bvh.export_compact())
+    for away in (1.0, 3.9, 4.1, 300.0, 1e3, 5e4, 1e5, 1e7):
+        _say(f"rays from far away: {away}")
+        rays = np.zeros((n, 8), np.float32)
+        rays[:, :3], rays[:, 4:7], rays[:, 7] = at - d * away, d, 1e20
+        want = _check(tt, oracle, scene, bvh, rays, f"{away} away", EXACT)
+        hit, _ = cb.trace(rays, any_hit=True, nthreads=8)
+        assert np.array_equal(scene.occluded(rays), (oracle.hit_ids(hit) >= 0).astype(np.int32))
+        ids, t, _, _ = scene.intersect(rays, tt.trace_cfg(1, 16, 128))
+        assert ((ids >= 0) == (oracle.hit_ids(want) >= 0)).all()
+        # noise of a computed distance off grazing rays: 1e-5 of the way
+        assert (np.abs(t - want[:, 1]) <= 1e-5 * want[:, 1]).mean() > 0.999
+    scene.close()
