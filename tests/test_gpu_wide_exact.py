@@ -235,3 +235,24 @@ def test_rays_from_far_away(tt, oracle, ctx):
         # noise of a computed distance off grazing rays: 1e-5 of the way
         assert (np.abs(t - want[:, 1]) <= 1e-5 * want[:, 1]).mean() > 0.999
     scene.close()
+
+
+@pytest.mark.parametrize("tris,mu,copies,flip", [(3000, 0.1, 2, False), (3000, 0.1, 3, True), (20000, 0.03, 2, True),
+                                                 (20000, 0.03, 5, False)])
+def test_coincident_triangles(tt, oracle, ctx, tris, mu, copies, flip):
+    """Every triangle several times, in shuffled order, with or without every other copy
+    facing the other way; large ones are split over several leaves. Exact ties are won by
+    the first triangle visited."""
+    _say(f"coincident triangles: {copies} of {tris}")
+    a = tt.Mesh.soup(tris, seed=6, mu=float(np.log(mu))).arrays()
+    t = np.concatenate([a["tris"][:, ::-1] if flip and k % 2 else a["tris"] for k in range(copies)])
+    t = t[np.random.default_rng(1).permutation(len(t))]
+    mesh = tt.Mesh.from_arrays(a["verts"], np.ascontiguousarray(t))
+    bvh = tt.BVH.build(mesh)
+    scene = tt.DeviceScene(ctx, mesh, bvh)
+    assert scene.walk()[0]
+    rays = np.concatenate([tt.rays_incoherent(mesh, 60000, seed=3),
+                           tt.rays_primary(200, 200, 1, (0.5, 0.5, -1.0), (0.5, 0.5, 0.0), seed=3)])
+    want = _check(tt, oracle, scene, bvh, rays, "coincident")
+    assert (oracle.hit_ids(want) >= 0).mean() > 0.3
+    scene.close()
