@@ -24,8 +24,7 @@
 // distance of the nearest other triangle (next_t): if it passes, the two-child walk enters
 // that leaf whatever its best distance was by then, and no tested triangle is nearer. If it
 // does not pass (a hit within rounding of its box's edge), or two triangles tie exactly
-// (the first one visited wins there) unless one comes directly after the other in all its
-// leaves, or the ray is one the quantised arithmetic does not
+// (the first one visited wins there) unless one is the other's twin (wide.hip), or the ray is one the quantised arithmetic does not
 // cover (non-finite or overflowing terms, negative tmin, a full stack), the lane walks the
 // two-child tree. An any-hit ray applies the leaf test to every triangle it would accept.
 // That rests on a culled box holding no triangle nearer than the best distance. In exact
@@ -265,10 +264,10 @@ __device__ __forceinline__ void walk_exact(const TraceArgs &a, int root, float o
     }
 }
 
-// Whether the two-child walk enters a leaf (its place: node * 2 + child, whatever the sign
-// bit) at best distance hit_t.
+// Whether the two-child walk enters a leaf (its place: node * 2 + child, below two other bits)
+// at best distance hit_t.
 __device__ __forceinline__ bool in_leaf(const TraceArgs &a, int place, const RayTerms &r, float hit_t) {
-    const float4 *np = a.nodes + (int64_t)((place & 0x7FFFFFFF) >> 1) * 4;
+    const float4 *np = a.nodes + (int64_t)((place & 0x3FFFFFFF) >> 1) * 4;
     const float4 xy = np[place & 1];
     const float2 z = reinterpret_cast<const float2 *>(np + 2)[place & 1];
     float e;
@@ -282,13 +281,19 @@ __device__ __forceinline__ bool in_leaf(const TraceArgs &a, int place, const Ray
 // Longer rings than the limit go to the full walk, which a lane alone takes some 150 us for:
 // with a limit of 16, exact camera rays on soup of 250k triangles took 418 or 585 us by the
 // rings' order, which differs from one build of the tree to the next; with 64, 415.
-__device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, const RayTerms &r, float t) {
+__device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, int chain, const RayTerms &r, float t,
+                                        float near) {
     if (in_leaf(a, place, r, t)) return true;
+    // (where another triangle as near is what keeps it out, that would do so elsewhere too)
+    if (t < near && in_leaf(a, place, r, near)) return false;
+    const auto word = [&](int at, int k) { return fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[k].w); };
+    // the leaf where the triangle was met last, if more than once
+    if (chain != rec && word(chain, 0) == word(rec, 0) && in_leaf(a, word(chain, 1), r, t)) return true;
     int at = rec;
     for (int i = 0; i < 64; ++i) {
-        at = fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[2].w) & 0x7FFFFFFF;
+        at = word(at, 2) & 0x7FFFFFFF;
         if (at == rec) return false;
-        if (in_leaf(a, fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)[1].w), r, t)) return true;
+        if (in_leaf(a, word(at, 1), r, t)) return true;
     }
     return false;
 }
@@ -299,22 +304,6 @@ __device__ __forceinline__ bool reached(const TraceArgs &a, int rec, int place, 
 __device__ __forceinline__ float noise_to(const TraceArgs &a, float dx, float dy, float dz, float t) {
     const float len = sqrtf(dx * dx + dy * dy + dz * dz);
     return len <= kUnitLength ? a.wide_noise * len * (t * len + a.wide_grain) : INFINITY;
-}
-
-// Whether triangle `id` is tested before that of a record wherever the latter is: a marked
-// record (mark: its second word's w) comes directly after the same triangle in all its leaves.
-// Such a triangle cannot take a ray from the other, so it does not count as another distance:
-// otherwise every hit on coincident triangles would end in a full walk (1.2M rays on soup of
-// 50k triangles, each twice: 2811 us, with this 906, once each 526; path tracing one with
-// faces on both sides 5818 and 3683; two-child loop 823 and 3544).
-__device__ __forceinline__ bool comes_after(const TraceArgs &a, uint32_t rec, int mark, int id) {
-    while (mark < 0) {
-        rec -= a.wide_step;
-        const float4 *tp = reinterpret_cast<const float4 *>(a.wide + rec);
-        if (fb(tp[0].w) == id) return true;
-        mark = fb(tp[1].w);
-    }
-    return false;
 }
 
 // The counts of the queue traced, uniform, and the slot of its r-th position (-1: none).
@@ -362,7 +351,7 @@ __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
 // lanes active), takes 1.43e9, 0.90e9 and 3.0 ms; each alone gains little, as the other
 // limit holds (four children in the while-while loop: 6.6 ms, slower).
 template <bool ANY, int S, int TRI, bool EXACT>
-__global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) {
+__global__ __launch_bounds__(256, ANY ? 1 : 6) void k_trace_wide(TraceArgs a) {
     static_assert(!EXACT || (!ANY && TRI == kTriReference), "kNoise is the reference test's");
     using E = typename std::conditional<ANY, int, uint64_t>::type;
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -434,6 +423,13 @@ __global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) 
     // the winner's record (-1: none; any hit: 0 once occluded). Its id and barycentrics go
     // straight to the ray's hit record when it is accepted, which frees their registers.
     int hit_rec = -1, hit_place = 0;   // (and the place of its leaf)
+    // A triangle tested after the winner wherever it is cannot take the ray from it, so its
+    // distance does not count: one whose twin (two bits of its record) is the winner, or was
+    // found to be so (chain). Otherwise every hit on coincident triangles would be a tie that
+    // ends in a full walk (1.2M rays on soup of 50k triangles, each twice: 2811 us, with this
+    // 599, once each 531; path tracing one with faces on both sides 5818 and 3589; two-child loop
+    // 823 and 3544). Also the winner itself where it was met again, in another leaf.
+    int chain = 0;
     float next_t = 0.0f;       // no other accepted triangle lies below this (at most where boxes are culled)
     bool redo = false;         // not for the wide walk
 
@@ -443,7 +439,8 @@ __global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) 
             const RayTerms r{idirx, idiry, idirz, ox * idirx, oy * idiry, oz * idirz, tmin};
             bool walk = redo;
             if (!ANY && !walk && hit_rec >= 0)
-                walk = !(hit_t < next_t) || !reached(a, hit_rec, hit_place, r, fminf(next_t, bf(cull)));
+                walk = !(hit_t < next_t) ||
+                       !reached(a, hit_rec, hit_place, chain, r, fminf(next_t, bf(cull)), hit_t * 1.00001f);
             if (walk) {
                 HitState h;
                 walk_exact<ANY, S, TRI>(a, a.roots ? a.roots[a.ray_root ? a.ray_root[rid] : 0] : 0, ox, oy, oz, dx, dy, dz,
@@ -653,13 +650,19 @@ __global__ __launch_bounds__(256, EXACT ? 6 : 1) void k_trace_wide(TraceArgs a) 
                         hit_t = t;
                         hit_rec = (int)rec;
                         hit_place = fb(B.w);
+                        chain = (int)rec;
                         cull = fb(t + t * spare);
                         if constexpr (EXACT) noise = min(noise, noise_to(a, dx, dy, dz, bf(cull)));
                     } else if (hit_rec >= 0 && t < next_t) {
-                        // Neither the same triangle again nor one that is never tested before it.
-                        // (Without a winner a triangle at or past tmax is no hit, and next_t is tmax.)
+                        // (without a winner a triangle at or past tmax is no hit, and next_t is tmax)
                         const int id = fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)hit_rec)->w);
-                        if (fb(A.w) != id && !comes_after(a, rec, fb(B.w), id)) next_t = fminf(next_t, t);
+                        const uint32_t twin = (uint32_t)fb(B.w) >> 30;
+                        const int at = (int)(rec - (twin & 1 ? a.wide_step : 0) - (twin & 2 ? 2 * a.wide_step : 0));
+                        if (fb(A.w) == id ||
+                            (twin && (at == chain ||
+                                      fb(reinterpret_cast<const float4 *>(a.wide + (uint32_t)at)->w) == id)))
+                            chain = (int)rec;
+                        else next_t = fminf(next_t, t);
                     }
                 }
             }

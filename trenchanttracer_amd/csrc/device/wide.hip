@@ -28,10 +28,11 @@
 // replaced by its own two while they fit (simulated on 1M-triangle soup: 24.2 visits of 3
 // loads per incoherent ray against 50.6 of 4; eight children with 80-byte nodes: 16.7
 // visits of 5). Triangle records are copied so that a node's leaves lie together; the
-// second word's w is the leaf's place in the two-child tree (node * 2 + child), negative where
-// the triangle comes directly after the same other one in each of its leaves (so that one is
-// tested first, always: what k_trace_wide needs to know of coincident triangles), the third's
+// second word's w is the leaf's place in the two-child tree (node * 2 + child), the third's
 // the next record of the same triangle (a ring over its leaves), negative at a leaf's end.
+// Above the place, two bits: 1 to 3 for a triangle that has a twin, which in each of its leaves
+// lies that many records before it (another number in another leaf), so that the twin is tested
+// before it, always. Triangles with equal centres, coincident ones, are made twins.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -46,7 +47,7 @@ namespace tt {
 namespace {
 
 constexpr int kMaxOffset = 127;   // largest unit offset of a slot
-constexpr int32_t kFirst = -2;              // no triangle id: the first of a leaf
+constexpr int32_t kNone = -2;               // no triangle id
 constexpr float kMaxSize = 1e30f;           // of sizes that exact hits are widened for
 constexpr int32_t kRingEnd = 0x7FFFFFFF;   // no unit index
 constexpr float kGrain = 0.25f;
@@ -78,7 +79,7 @@ struct WideBuild {
     int32_t *parent;        // of a listed node, its parent's place in the list (roots: -1)
     int32_t *size;          // ... bits of its triangles' largest size (-1: no triangle)
     int32_t *last_of;       // [triangle id]: first unit of its record linked last, or -1
-    int32_t *after;         // ... the triangle before it in its leaves, kFirst where they differ, or -1
+    int32_t *twin;          // ... the one before it, kNone where its leaves have none or others, or -1
     int32_t ids;            // triangle ids below this have a ring; others stand alone
     WideState *state;
     int32_t node_cap, rec_cap;
@@ -159,10 +160,16 @@ __device__ int wave_scan(int v, int *total) {   // exclusive sum over the wave's
     return s - v;
 }
 
+// Equal to the rounding of its terms.
+__device__ bool near(float x, float y, float v, float a, float b) {
+    return fabsf(x - y) <= 0x1p-20f * (fabsf(v) + fabsf(a) + fabsf(b));
+}
+
 // (returns the largest size)
 __device__ float copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32_t place, int32_t at, bool last) {
     float size = 0.0f;
-    int32_t before = kFirst;
+    float3 centre[3];   // of the last three, the latest first
+    int32_t ids[3] = {-1, -1, -1};
     const float4 *t = b.tris + (int64_t)~ref * 3;
     for (int i = 0; i < count; ++i) {
         const int32_t unit = b.step * (at + i);
@@ -177,12 +184,31 @@ __device__ float copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32
         // the record before this one in the ring; the first closes it (k_wide_rings)
         int32_t link = id >= 0 && id < b.ids ? atomicExch(&b.last_of[id], unit) : unit;
         if (link < 0) link = kRingEnd;
+        // (three times the centre; v0 + v0 + v0 + e1 + e2 whichever vertex comes first)
+        const float4 v0 = t[3 * i];
+        const float3 c = make_float3(3.0f * v0.x + (e1.x + e2.x), 3.0f * v0.y + (e1.y + e2.y), 3.0f * v0.z + (e1.z + e2.z));
+        uint32_t back = 0;
+        int32_t twin = kNone;
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+            if (ids[k] >= 0 && near(c.x, centre[k].x, v0.x, e1.x, e2.x) && near(c.y, centre[k].y, v0.y, e1.y, e2.y) &&
+                near(c.z, centre[k].z, v0.z, e1.z, e2.z)) {
+                back = k + 1;
+                twin = ids[k];
+            }
         if (id >= 0 && id < b.ids) {
-            const int32_t was = atomicCAS(&b.after[id], -1, before);
-            if (was != -1 && was != before) atomicExch(&b.after[id], kFirst);
+            const int32_t was = atomicCAS(&b.twin[id], -1, twin);
+            if (was != -1 && was != twin) atomicExch(&b.twin[id], kNone);
+        } else {
+            back = 0;
         }
-        before = id >= 0 ? id : kFirst;
-        e1.w = __int_as_float(place);
+        for (int k = 2; k > 0; --k) {
+            centre[k] = centre[k - 1];
+            ids[k] = ids[k - 1];
+        }
+        centre[0] = c;
+        ids[0] = id;
+        e1.w = __int_as_float(place | (int32_t)(back << 30));
         e2.w = __int_as_float(link | (last && i + 1 == count ? (int32_t)0x80000000 : 0));
         to[0] = t[3 * i];
         to[1] = e1;
@@ -192,17 +218,17 @@ __device__ float copy_leaf(const WideBuild &b, int32_t ref, int32_t count, int32
 }
 
 // Closes the rings: the record linked first (it holds kRingEnd) points to the one linked
-// last. One thread per triangle id, which follows its ring to that record, and marks the
-// triangle's records if it always comes after the same one.
+// last. One thread per triangle id, which follows its ring to that record, and clears the twin
+// bits of a triangle that has not the same one in all its leaves.
 __global__ __launch_bounds__(256) void k_wide_rings(WideBuild b) {
     const int32_t id = blockIdx.x * 256 + threadIdx.x;
     if (id >= b.ids || b.last_of[id] < 0) return;
     const int32_t last = b.last_of[id];
-    const bool after = b.after[id] >= 0;
+    const bool twin = b.twin[id] >= 0;
     for (int32_t at = last;;) {
         int32_t *link = reinterpret_cast<int32_t *>(b.wide + at + 2) + 3;
         const int32_t v = *link;
-        if (after) *(link - 4) |= (int32_t)0x80000000;
+        if (!twin) *(link - 4) &= 0x3FFFFFFF;
         if ((v & 0x7FFFFFFF) == kRingEnd) {
             *link = last | (v & (int32_t)0x80000000);
             return;
@@ -512,8 +538,8 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     b.parent = reinterpret_cast<int32_t *>(b.list + nodes);
     b.size = b.parent + nodes;
     b.last_of = b.size + nodes;
-    b.after = b.last_of + ids;
-    int32_t *d_roots = b.after + ids;
+    b.twin = b.last_of + ids;
+    int32_t *d_roots = b.twin + ids;
     b.roots = d_roots;
     b.step = step;
     b.nroots = (int32_t)roots.size();
@@ -536,7 +562,7 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
     hipError_t err = hipMemcpyAsync(b.state, &state, sizeof(state), hipMemcpyHostToDevice, hs);
     if (err == hipSuccess) err = hipMemcpyAsync(d_roots, roots.data(), root_bytes, hipMemcpyHostToDevice, hs);
     if (err == hipSuccess) {
-        const int64_t words = 2 * ((int64_t)nodes + ids);   // parent, size, last_of, after
+        const int64_t words = 2 * ((int64_t)nodes + ids);   // parent, size, last_of, twin
         hipLaunchKernelGGL(k_wide_clear, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, hs, b.parent, words);
         err = hipGetLastError();
     }
