@@ -413,7 +413,7 @@ __global__ __launch_bounds__(64) void k_wide_level(WideBuild b, int32_t first, i
 // The levels from the roots down to the first with more nodes than one block has threads. A
 // launch for each level, with its count read back, takes about 20 us more: creating a scene of
 // 300 triangles 395 us, with this 321 (104 without the tree), of 2000 718 and 617, of 250k
-// 12511 and 12337.
+// 12511 and 12337 (12078 with the sums of k_wide_sizes added by block).
 constexpr int kTopThreads = 1024;
 __global__ __launch_bounds__(kTopThreads) void k_wide_top(WideBuild b) {
     int32_t first = 0, count = b.nroots;
@@ -428,14 +428,19 @@ __global__ __launch_bounds__(kTopThreads) void k_wide_top(WideBuild b) {
     if (threadIdx.x == 0) b.state->built = first;
 }
 
-// Every node's size code into its record, and the cost of boxes widened by it.
+// Every node's size code into its record, and the cost of boxes widened by it. Bound by the
+// atomic adds to the sums (13 ns each), so at most 256 blocks walk the nodes and add once each
+// (200,000 nodes, a wave's sums added on their own: 305 us, with this 26).
+constexpr int kSizeBlocks = 256;
 __global__ __launch_bounds__(256) void k_wide_sizes(WideBuild b, int32_t count) {
-    const int32_t i = blockIdx.x * 256 + threadIdx.x;
+    __shared__ unsigned long long sum[2 + kReaches];
+    if (threadIdx.x < 2 + kReaches) sum[threadIdx.x] = 0;
+    __syncthreads();
     float most = 0.0f;
     for (int32_t k = 0; k < b.nroots; ++k) most = fmaxf(most, __int_as_float(max(b.size[k], 0)));
+    if (blockIdx.x == 0 && threadIdx.x == 0) b.state->most = most;
     unsigned long long cost[2 + kReaches] = {};
-    if (i < count) {
-        if (i == 0) b.state->most = most;
+    for (int32_t i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) {
         uint4 *w = b.wide + b.step * (i < b.nroots ? i : b.list[i].x);
         const uint4 q = w[1], r = w[2];
         const float share = __int_as_float(max(b.size[i], 0)) / most;
@@ -461,8 +466,10 @@ __global__ __launch_bounds__(256) void k_wide_sizes(WideBuild b, int32_t count) 
 #pragma unroll
     for (int f = 0; f < 2 + kReaches; ++f) {
         for (int o = 32; o > 0; o >>= 1) cost[f] += __shfl_down(cost[f], o);
-        if (__lane_id() == 0 && cost[f]) atomicAdd(&b.state->cost[f], cost[f]);
+        if (__lane_id() == 0) atomicAdd(&sum[f], cost[f]);
     }
+    __syncthreads();
+    if (threadIdx.x < 2 + kReaches) atomicAdd(&b.state->cost[threadIdx.x], sum[threadIdx.x]);
 }
 
 // Whether a random line through the tree's root box is expected to cost more than `limit`
@@ -605,7 +612,8 @@ tt_status build_wide(tt_scene *s, const std::vector<int32_t> &dev_nodes, const s
         if (err == hipSuccess) err = hipStreamSynchronize(hs);
     }
     if (err == hipSuccess && state.unfit == 0) {
-        hipLaunchKernelGGL(k_wide_sizes, dim3((unsigned)((state.nodes + 255) / 256)), dim3(256), 0, hs, b, state.nodes);
+        hipLaunchKernelGGL(k_wide_sizes, dim3((unsigned)std::min((state.nodes + 255) / 256, kSizeBlocks)), dim3(256), 0, hs, b,
+                           state.nodes);
         if (ids > 0) hipLaunchKernelGGL(k_wide_rings, dim3((unsigned)((ids + 255) / 256)), dim3(256), 0, hs, b);
         err = hipGetLastError();
         if (err == hipSuccess) err = hipMemcpyAsync(&state, b.state, sizeof(state), hipMemcpyDeviceToHost, hs);
