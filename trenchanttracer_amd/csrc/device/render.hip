@@ -1129,8 +1129,8 @@ __global__ __launch_bounds__(256) void k_guide_slots(const uint64_t *mask, const
 
 // GUIDED: the guide's mixture, training records and roulette rule are compiled in
 // only for guided renders, so the plain kernel keeps its registers for occupancy.
-// Bound by HBM and, on the camera bounce, by VALU issue about equally (133M camera-bounce
-// paths: 77% of the issue slots, 3 TB/s), so a path's bytes are kept down: the throughput
+// Bound by VALU issue (133M camera-bounce paths 91% of the slots and 4.6 TB/s, the next bounce
+// 93% and 2.8; before the bytes went down 77% and 3 TB/s), so a path's bytes are kept down: the throughput
 // travels with the ray by queue slot (read and written in order), the radiance is touched
 // only where a bounce adds some, the scene of a ray comes from its path id and is queued
 // for the traversal only when there are several, and the camera bounce's path ids are not

@@ -339,9 +339,9 @@ __device__ __forceinline__ int group_bits(uint32_t n, int32_t spread) {
     return full ? min(6, 32 - __clz((int)full)) : 0;
 }
 
-// EXACT widens boxes as kNoise asks (9 instructions a node, 73 VGPRs as held to 6 waves per
-// SIMD, 82 without): soup of 250k triangles, 1.2M rays, 634 us as variant 1, 678 exact, of 20k
-// 448 and 506; with nothing to widen, 634 and 448.
+// EXACT widens boxes as kNoise asks (9 instructions a node, 78 VGPRs as held to 6 waves per
+// SIMD, 87 without): whole calls of 1.2M rays, soup of 250k triangles, 720 us as variant 1, 746
+// exact, of 20k 378 and 383.
 //
 // Four-child walk. What bounds it: VALU issue first, vector memory lane loads second. On
 // the 1M-triangle soup (8.3M rays in Morton order) the two-child while-while loop kept VALU
